@@ -427,14 +427,15 @@ MOE_DEV void route_row(const float* row, int t, int E, int k, float tau,
   for (int i = 0; i < EPL; ++i) {
     const int e = lane + 64 * i;
     v[i] = e < E ? row[e] : -INFINITY;
-    if (e < E) mx = fmaxf(mx, v[i] / tau);
+    ex[i] = v[i] / tau;
+    if (e < E) mx = fmaxf(mx, ex[i]);
   }
   mx = wave_max(mx);
   float s = 0.0f;
 #pragma unroll
   for (int i = 0; i < EPL; ++i) {
     const int e = lane + 64 * i;
-    ex[i] = e < E ? expf(v[i] / tau - mx) : 0.0f;
+    ex[i] = e < E ? expf(ex[i] - mx) : 0.0f;
     s += ex[i];
   }
   s = wave_sum(s);
@@ -446,41 +447,35 @@ MOE_DEV void route_row(const float* row, int t, int E, int k, float tau,
   }
   if (lane == 0) lse[t] = mx + logf(s);
 
+  // Selection j: the wave maximum of the candidates left, then the lowest
+  // expert that holds it (one ballot per 64 experts, lowest block first).
   uint32_t taken = 0;
+#pragma unroll
+  for (int i = 0; i < EPL; ++i) {
+    if (isnan(v[i])) v[i] = -INFINITY;
+    if (lane + 64 * i >= E) taken |= 1u << i;
+  }
   float wsel = 0.0f;
   sel = -1;
   float wsum = 0.0f;
   for (int j = 0; j < k; ++j) {
     float bv = -INFINITY;
-    int be = INT_MAX;
-#pragma unroll
-    for (int i = 0; i < EPL; ++i) {
-      const int e = lane + 64 * i;
-      const float val = isnan(v[i]) ? -INFINITY : v[i];
-      if (e < E && !((taken >> i) & 1u) && (be == INT_MAX || val > bv)) {
-        bv = val;
-        be = e;
-      }
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const float ov = __shfl_xor(bv, o, 64);
-      const int oe = __shfl_xor(be, o, 64);
-      const bool better = oe != INT_MAX && (be == INT_MAX || ov > bv || (ov == bv && oe < be));
-      if (better) {
-        bv = ov;
-        be = oe;
-      }
-    }
-    // every lane now holds the same winner; its owner marks it taken
-    float mine = 0.0f;
 #pragma unroll
     for (int i = 0; i < EPL; ++i)
-      if (lane + 64 * i == be) {
-        taken |= 1u << i;
+      if (!((taken >> i) & 1u)) bv = fmaxf(bv, v[i]);
+    bv = wave_max(bv);
+    int be = -1;
+    float mine = 0.0f;
+#pragma unroll
+    for (int i = 0; i < EPL; ++i) {
+      const uint64_t m = __ballot(!((taken >> i) & 1u) && v[i] == bv);
+      if (be < 0 && m != 0) {  // wave-uniform
+        be = 64 * i + __ffsll((unsigned long long)m) - 1;
         mine = ex[i];
+        if (lane == (be & 63)) taken |= 1u << i;
       }
-    const float pj = __shfl(mine, be & 63, 64) / s;
+    }
+    const float pj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), be & 63)) / s;
     if (lane == j) {
       wsel = pj;
       sel = be;
@@ -1488,13 +1483,6 @@ __global__ __launch_bounds__(256) void k_combine_bwd(const T* __restrict__ dout,
   }
 }
 
-// v of lane l ^ X within each group of four lanes (DPP quad_perm, X = 1 or 2).
-template <int X>
-MOE_DEV float quad_xor(float v) {
-  constexpr int ctrl = X == 1 ? 0xB1 : 0x4E;  // quad_perm [1,0,3,2] / [2,3,0,1]
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xF, 0xF, false));
-}
-
 // ------------------------------------------------------------------ expert GEMMs (backward)
 // dA = alpha * dY Wd (NN, K = H), then the SwiGLU backward in the epilogue:
 // dG = dA * U * silu'(G), dU = dA * silu(G).
@@ -1575,8 +1563,8 @@ __global__ __launch_bounds__(C::THREADS) void k_down_dgrad(const T* __restrict__
       if constexpr (GROUPED) {
         // the row's 4 lanes (lane / 4 equal) hold its 32-column block; DPP
         // quad permutes (lanes xor 1, then xor 2) keep the sum off the LDS
-        const float p1 = part + quad_xor<1>(part);
-        const float p2 = quad_xor<2>(p1);
+        const float p1 = part + lane_xor<1>(part);
+        const float p2 = lane_xor<2>(p1);
         const bool lo = (threadIdx.x & 2) == 0;
         const float blk = lo ? p1 + p2 : p2 + p1;
         if (m < mv && (threadIdx.x & 3) == 0 && n0 + n < N)
