@@ -95,16 +95,17 @@ MOE_DEV float sigmoid_f(float g) { return 1.0f / (1.0f + __expf(-g)); }
 // v of lane l ^ X (X = 1, 2, 4 or 8), without the LDS crossbar: DPP quad
 // permutes, row shifts by four masked to alternating banks, a row rotation.
 template <int X>
-MOE_DEV float lane_xor(float v) {
+MOE_DEV int lane_xor(int i) {
   static_assert(X == 1 || X == 2 || X == 4 || X == 8, "inside a row of 16 lanes");
-  const int i = __float_as_int(v);
-  if constexpr (X == 1) return __int_as_float(__builtin_amdgcn_update_dpp(0, i, 0xB1, 0xF, 0xF, false));
-  if constexpr (X == 2) return __int_as_float(__builtin_amdgcn_update_dpp(0, i, 0x4E, 0xF, 0xF, false));
-  if constexpr (X == 8) return __int_as_float(__builtin_amdgcn_update_dpp(0, i, 0x128, 0xF, 0xF, false));
+  if constexpr (X == 1) return __builtin_amdgcn_update_dpp(0, i, 0xB1, 0xF, 0xF, true);
+  if constexpr (X == 2) return __builtin_amdgcn_update_dpp(0, i, 0x4E, 0xF, 0xF, true);
+  if constexpr (X == 8) return __builtin_amdgcn_update_dpp(0, i, 0x128, 0xF, 0xF, true);
   // lanes 0-3 and 8-11 of a row read four lanes up, the others four down
   const int up = __builtin_amdgcn_update_dpp(0, i, 0x104, 0xF, 0x5, false);
-  return __int_as_float(__builtin_amdgcn_update_dpp(up, i, 0x114, 0xF, 0xA, false));
+  return __builtin_amdgcn_update_dpp(up, i, 0x114, 0xF, 0xA, false);
 }
+template <int X>
+MOE_DEV float lane_xor(float v) { return __int_as_float(lane_xor<X>(__float_as_int(v))); }
 
 // Wave-wide (64 lanes) butterfly reductions over lane distances 32, 16, ... 1:
 // fixed order, so bit-reproducible.  Distances 32 and 16 exchange register
@@ -114,14 +115,14 @@ MOE_DEV float lane_xor(float v) {
 // of these and k more for the top-k, each a serial chain: a forward of one
 // token (H = 2048, E = 64, k = 6) 101.2 -> 98.9 us, of 64 (E = 128, k = 8)
 // 862 -> 855 us, the same bits.
-template <class OP>
-MOE_DEV float wave_butterfly(float v, OP&& op) {
-  uint32_t u = __float_as_uint(v);
+template <class T, class OP>
+MOE_DEV T wave_butterfly(T v, OP&& op) {
+  uint32_t u = __builtin_bit_cast(uint32_t, v);
   auto s = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  v = op(__uint_as_float(s[0]), __uint_as_float(s[1]));
-  u = __float_as_uint(v);
+  v = op(__builtin_bit_cast(T, (uint32_t)s[0]), __builtin_bit_cast(T, (uint32_t)s[1]));
+  u = __builtin_bit_cast(uint32_t, v);
   s = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  v = op(__uint_as_float(s[0]), __uint_as_float(s[1]));
+  v = op(__builtin_bit_cast(T, (uint32_t)s[0]), __builtin_bit_cast(T, (uint32_t)s[1]));
   v = op(v, lane_xor<8>(v));
   v = op(v, lane_xor<4>(v));
   v = op(v, lane_xor<2>(v));
@@ -132,6 +133,9 @@ MOE_DEV float wave_sum(float v) {
 }
 MOE_DEV float wave_max(float v) {
   return wave_butterfly(v, [](float a, float b) { return fmaxf(a, b); });
+}
+MOE_DEV int wave_max(int v) {
+  return wave_butterfly(v, [](int a, int b) { return a > b ? a : b; });
 }
 
 // Map workgroup b to a logical tile id in [0, n) so that the blocks one XCD

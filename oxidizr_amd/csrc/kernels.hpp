@@ -94,8 +94,8 @@ struct RowGroups {
 // scalar registers so that the address arithmetic built on them stays scalar.
 MOE_DEV int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// Waves of the router kernels that split the hidden dimension (k_router_small,
-// k_router_route).
+// Parts the router kernels split the hidden dimension into (k_small_front, two
+// per wave; k_router_route, one).
 constexpr int kRouterWaves = 16;
 
 // 16 x 16 x 32 bf16 MFMA: acc[r] of lane l = sum_k a[row 4 (l / 16) + r][k] * b[row l % 16][k]
@@ -411,31 +411,49 @@ __global__ __launch_bounds__(256) void k_router_reduce(const float* __restrict__
 // `row` holds the token's E logits (global memory, or a row staged in LDS by
 // the fused router kernel): the same arithmetic either way, so the same bits.
 // Also returns, in registers, the lane's probabilities pr[i] (expert
-// lane + 64 i, 0 past E) and, in lane j < k, the j-th chosen expert (sel;
-// -1 in lanes >= k).  Selection j is kept by lane j rather than in arrays
-// indexed by the runtime k, which the compiler would keep in scratch or in
-// 48 extra registers.
+// lane + 64 i, 0 past E), the log-sum-exp and, in lane j < k, the j-th chosen
+// expert (sel; -1 in lanes >= k).  Selection j is kept by lane j rather than in
+// arrays indexed by the runtime k, which the compiler would keep in scratch or
+// in 48 extra registers.
+//
+// The top-k compares integer keys that order as the floats do (-0 as +0, NaN as
+// -inf; a taken or absent expert holds INT_MIN, below every key): an integer
+// maximum takes its DPP operand directly and needs no NaN canonicalisation, so
+// a selection is about 25 instructions.  A CU that routes 64 tokens (16 waves,
+// k_small_route) is bound by their number: 64 tokens, E = 64, k = 6, 18.5 ->
+// 14.6 us; E = 128, k = 8, 26.6 -> 17.5 us.
+MOE_DEV int route_key(float f) {
+  const int i = __float_as_int(isnan(f) ? -INFINITY : f + 0.0f);
+  return i ^ ((i >> 31) & 0x7fffffff);
+}
 template <int EPL>
 MOE_DEV void route_row(const float* row, int t, int E, int k, float tau,
                        int norm, float* __restrict__ probs, float* __restrict__ lse,
                        int* __restrict__ idx, float* __restrict__ w, float (&pr)[EPL],
-                       int& sel) {
+                       int& sel, float& lse_t) {
   const int lane = threadIdx.x & 63;
-  float v[EPL], ex[EPL];
+  float ex[EPL];
+  int key[EPL];
   float mx = -INFINITY;
 #pragma unroll
   for (int i = 0; i < EPL; ++i) {
     const int e = lane + 64 * i;
-    v[i] = e < E ? row[e] : -INFINITY;
-    ex[i] = v[i] / tau;
-    if (e < E) mx = fmaxf(mx, ex[i]);
+    const float v = e < E ? row[e] : -INFINITY;
+    key[i] = e < E ? route_key(v) : INT_MIN;
+    ex[i] = v;
   }
+  if (tau != 1.0f) {  // x / 1 is x
+#pragma unroll
+    for (int i = 0; i < EPL; ++i) ex[i] /= tau;
+  }
+#pragma unroll
+  for (int i = 0; i < EPL; ++i)
+    if (lane + 64 * i < E) mx = fmaxf(mx, ex[i]);
   mx = wave_max(mx);
   float s = 0.0f;
 #pragma unroll
   for (int i = 0; i < EPL; ++i) {
-    const int e = lane + 64 * i;
-    ex[i] = e < E ? expf(ex[i] - mx) : 0.0f;
+    ex[i] = lane + 64 * i < E ? expf(ex[i] - mx) : 0.0f;
     s += ex[i];
   }
   s = wave_sum(s);
@@ -445,37 +463,31 @@ MOE_DEV void route_row(const float* row, int t, int E, int k, float tau,
     pr[i] = e < E ? ex[i] / s : 0.0f;
     if (e < E) probs[(int64_t)t * E + e] = pr[i];
   }
-  if (lane == 0) lse[t] = mx + logf(s);
+  lse_t = mx + logf(s);
+  if (lane == 0) lse[t] = lse_t;
 
-  // Selection j: the wave maximum of the candidates left, then the lowest
-  // expert that holds it (one ballot per 64 experts, lowest block first).
-  uint32_t taken = 0;
-#pragma unroll
-  for (int i = 0; i < EPL; ++i) {
-    if (isnan(v[i])) v[i] = -INFINITY;
-    if (lane + 64 * i >= E) taken |= 1u << i;
-  }
+  // Selection j: the wave maximum of the keys left, then the lowest expert
+  // that holds it (one ballot per 64 experts, lowest block first).
   float wsel = 0.0f;
   sel = -1;
   float wsum = 0.0f;
   for (int j = 0; j < k; ++j) {
-    float bv = -INFINITY;
+    int bk = key[0];
 #pragma unroll
-    for (int i = 0; i < EPL; ++i)
-      if (!((taken >> i) & 1u)) bv = fmaxf(bv, v[i]);
-    bv = wave_max(bv);
+    for (int i = 1; i < EPL; ++i) bk = max(bk, key[i]);
+    bk = wave_max(bk);
     int be = -1;
     float mine = 0.0f;
 #pragma unroll
     for (int i = 0; i < EPL; ++i) {
-      const uint64_t m = __ballot(!((taken >> i) & 1u) && v[i] == bv);
+      const uint64_t m = __ballot(key[i] == bk);
       if (be < 0 && m != 0) {  // wave-uniform
         be = 64 * i + __ffsll((unsigned long long)m) - 1;
-        mine = ex[i];
-        if (lane == (be & 63)) taken |= 1u << i;
+        mine = pr[i];
+        if (lane == (be & 63)) key[i] = INT_MIN;
       }
     }
-    const float pj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), be & 63)) / s;
+    const float pj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), be & 63));
     if (lane == j) {
       wsel = pj;
       sel = be;
@@ -496,9 +508,9 @@ __global__ __launch_bounds__(256) void k_route(const float* __restrict__ logits,
                                                int* __restrict__ idx, float* __restrict__ w) {
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= Tn) return;
-  float pr[EPL];
+  float pr[EPL], l;
   int sel;
-  route_row<EPL>(logits + (int64_t)t * E, t, E, k, tau, norm, probs, lse, idx, w, pr, sel);
+  route_row<EPL>(logits + (int64_t)t * E, t, E, k, tau, norm, probs, lse, idx, w, pr, sel, l);
 }
 
 // ------------------------------------------------------------------ fused router
@@ -586,9 +598,9 @@ __global__ __launch_bounds__(64 * kRouterWaves) __attribute__((amdgpu_waves_per_
   if (wave < ntok) {
     const int t = t0 + wave;
     for (int e = lane; e < E; e += 64) logits[(int64_t)t * E + e] = lg[wave][e];
-    float pr[1];
+    float pr[1], l;
     int sel;
-    route_row<1>(&lg[wave][0], t, E, k, tau, norm, probs, lse, idx, w, pr, sel);
+    route_row<1>(&lg[wave][0], t, E, k, tau, norm, probs, lse, idx, w, pr, sel, l);
     pl[wave][lane] = pr[0];
     if (lane < k) atomicAdd(&hist[sel], 1);
   }
@@ -641,9 +653,9 @@ __global__ __launch_bounds__(1024) void k_reduce_route(
   __syncthreads();
   if (wave < ntok) {
     const int t = t0 + wave;
-    float pr[EPL];
+    float pr[EPL], l;
     int sel;
-    route_row<EPL>(&lg[wave][0], t, E, k, tau, norm, probs, lse, idx, w, pr, sel);
+    route_row<EPL>(&lg[wave][0], t, E, k, tau, norm, probs, lse, idx, w, pr, sel, l);
 #pragma unroll
     for (int i = 0; i < EPL; ++i) pl[wave][lane + 64 * i] = pr[i];
     if (lane < k) atomicAdd(&hist[sel], 1);
@@ -743,6 +755,10 @@ __global__ __launch_bounds__(256) void k_losses(const float* __restrict__ P,
 }
 
 // ------------------------------------------------------------------ dispatch
+// Batches of up to this many tokens are routed and dispatched by one workgroup
+// (k_small_route).
+constexpr int kRouteSmallTokens = 64;
+
 // Per-block expert histogram of 256 tokens' k assignments.
 __global__ __launch_bounds__(256) void k_hist(const int* __restrict__ idx, int Tn, int k, int E,
                                               int* __restrict__ block_hist) {
@@ -966,75 +982,6 @@ __global__ __launch_bounds__(256) void k_scatter(const int* __restrict__ idx, in
     const int pos = block_base[(int64_t)blockIdx.x * E + e] + wbase[wave * E + e] + rank;
     perm[pos] = t * k + j;
     inv_perm[(int64_t)t * k + j] = pos;
-  }
-}
-
-// Dispatch of a small batch (T <= kRouteSmallTokens, after k_route) in one
-// workgroup of 1024 threads, with the bits of the multi-kernel path: P is
-// summed in k_colsum_partial's order (four running sums over t mod 4, added
-// in order, one lane each) and scaled as k_colsum_final does; counts,
-// offsets and tile prefixes come from scan_counts; the rank of assignment
-// (t, j) within its expert is the number of earlier tokens that chose the
-// expert, read from a 64-bit token mask per expert (built with LDS atomic
-// ORs, which do not depend on order).
-constexpr int kRouteSmallTokens = 64;
-__global__ __launch_bounds__(1024) void k_dispatch_small(const int* __restrict__ idx,
-                                                         const float* __restrict__ probs, int Tn,
-                                                         int E, int k, float scale,
-                                                         float* __restrict__ P,
-                                                         int* __restrict__ counts,
-                                                         int* __restrict__ offsets,
-                                                         int* __restrict__ tile_prefix,
-                                                         int* __restrict__ perm,
-                                                         int* __restrict__ inv_perm) {
-  __shared__ int sidx[kRouteSmallTokens * 16];
-  __shared__ unsigned tmask[1024][2];
-  __shared__ int cnt[1024], offs[1024], wsum[16 * kScanCount];
-  const int tid = threadIdx.x;
-  for (int e = tid; e < E; e += 1024) tmask[e][0] = tmask[e][1] = 0u;
-  for (int i = tid; i < Tn * k; i += 1024) sidx[i] = idx[i];
-  // P: lanes 4e + q hold the running sum over tokens t = q mod 4
-  for (int e0 = 0; e0 < E; e0 += 256) {
-    const int e = e0 + (tid >> 2), q = tid & 3;
-    float r = 0.0f;
-    if (e < E) {
-      float v[kRouteSmallTokens / 4];
-#pragma unroll
-      for (int i = 0; i < kRouteSmallTokens / 4; ++i) {
-        const int t = q + 4 * i;
-        v[i] = t < Tn ? probs[(int64_t)t * E + e] : 0.0f;
-      }
-#pragma unroll
-      for (int i = 0; i < kRouteSmallTokens / 4; ++i)
-        if (q + 4 * i < Tn) r += v[i];
-    }
-    const int base = threadIdx.x & 60;  // lanes 4e .. 4e + 3 of this wave
-    const float r0 = __shfl(r, base, 64), r1 = __shfl(r, base + 1, 64);
-    const float r2 = __shfl(r, base + 2, 64), r3 = __shfl(r, base + 3, 64);
-    // k_colsum_final adds this single partial to three zeros: the same value
-    if (e < E && q == 0) P[e] = (((r0 + r1) + r2) + r3) * scale;
-  }
-  __syncthreads();
-  for (int i = tid; i < Tn * k; i += 1024) {
-    const int t = i / k;
-    atomicOr(&tmask[sidx[i]][t >> 5], 1u << (t & 31));
-  }
-  __syncthreads();
-  if (tid < E) {
-    const int c = __popc(tmask[tid][0]) + __popc(tmask[tid][1]);
-    cnt[tid] = c;
-    counts[tid] = c;
-  }
-  __syncthreads();
-  scan_counts(cnt, E, offsets, tile_prefix, offs, wsum);
-  for (int i = tid; i < Tn * k; i += 1024) {
-    const int t = i / k, e = sidx[i];
-    const unsigned lo = tmask[e][0], hi = tmask[e][1];
-    const int rank = t < 32 ? __popc(lo & ((1u << t) - 1u))
-                            : __popc(lo) + __popc(hi & ((1u << (t - 32)) - 1u));
-    const int pos = offs[e] + rank;
-    perm[pos] = i;
-    inv_perm[i] = pos;
   }
 }
 
@@ -2127,26 +2074,16 @@ __global__ __launch_bounds__(256) void k_rowsum(const float* __restrict__ in, in
 
 // ------------------------------------------------------------------ small-token forward
 // With T <= kSkinnyMaxTokens no expert holds more than that many rows, and the
-// forward is a stream of the touched experts' weights.  One wave owns 16 weight
-// rows and multiplies them with every token row of the expert (up to four
-// chunks of 16) using v_mfma_f32_16x16x32_bf16, A = token rows, B = weight
-// rows.  In a 256-wide k-chunk, MFMA step q covers k = 256 kc + 32 q + [0, 32):
-// lane l (row l % 16, group g = l / 16) supplies k-vector 32 q + 8 g of its
-// weight row and of its token row, so the four lanes of a row read 64
-// contiguous bytes per load instruction.  Experts without tokens read
-// no weights.  GATEUP: out0 = G, out1 = U, out2 = silu(G) * U from W0 = W_g,
-// W1 = W_u (out0 and out1 skipped when out0 is null); otherwise out0 = X W0^T
-// (down projection).
+// forward is a stream of the touched experts' weights.  A wave multiplies 16
+// weight rows with every token row of the expert (up to four chunks of 16)
+// using v_mfma_f32_16x16x32_bf16, A = token rows, B = weight rows.  In a
+// 256-wide k-chunk, MFMA step q covers k = 256 kc + 32 q + [0, 32): lane l
+// (row l % 16, group g = l / 16) supplies k-vector 32 q + 8 g of its weight row
+// and of its token row, so the four lanes of a row read 64 contiguous bytes
+// per load instruction.  GATEUP: out0 = G, out1 = U, out2 = silu(G) * U from
+// W0 = W_g, W1 = W_u (out0 and out1 skipped when out0 is null); otherwise
+// out0 = X W0^T (down projection).
 constexpr int kSkinnyMaxTokens = 64;
-constexpr int kSkinnyRows = 64;  // weight rows (output columns) per workgroup
-// Dynamic LDS every launch of the narrow (<= 16 tokens per expert) kernels
-// reserves, unused by the kernel: half of a CU's 160 KB, so a CU holds two
-// workgroups (two waves per SIMD) instead of the five its registers allow.
-// Fewer concurrent weight streams read HBM faster: config 4's gate/up stream
-// 69.8-70.2 % -> 71.4-72.0 % of 8 TB/s over four runs each (one workgroup per
-// CU: 70.6 %; prefetching the next k-chunk at two: 68.1-68.4 %).
-constexpr int kSkinnyLdsReserve = 80 * 1024;
-
 
 // A pointer every lane holds, moved to scalar registers: buffer resources
 // built from it then stay scalar (a resource the compiler cannot prove uniform
@@ -2159,96 +2096,85 @@ MOE_DEV const T* uni_ptr(const T* p) {
   return (const T*)(((uint64_t)hi << 32) | lo);
 }
 
-// The expert holding the j-th (from 0) group of more than 16 rows, or -1:
-// each wave counts the wide groups 64 at a time with a ballot.  Uniform.
-MOE_DEV int nth_wide_group(const int* offsets, int G, int j) {
-  const int lane = threadIdx.x & 63;
-  int seen = 0;
-  for (int base = 0; base < G; base += 64) {
-    const int e = base + lane;
-    const bool wide = e < G && offsets[e + 1] - offsets[e] > 16;
-    uint64_t m = __ballot(wide);
-    const int n = __popcll(m);
-    if (j < seen + n) {
-      for (int i = seen; i < j; ++i) m &= m - 1;  // drop the lower wide groups
-      return uni(base + __ffsll((unsigned long long)m) - 1);
-    }
-    seen += n;
-  }
-  return -1;
-}
-// Routed launches of the WIDE kernel need blocks for at most this many groups.
-inline int max_wide_groups(int64_t rows, int G) {
-  const int64_t w = rows / 17;
-  return (int)(w < G ? w : G);
-}
+// One expert of a small batch: its rows [r0, r0 + rows) of the permutation and
+// its weights.  The routing writes one per touched expert, experts ascending
+// (rows = 0 in the rest of the list), so that the workgroups of a launch are
+// those with work and each finds all it needs with one load.
+struct SkinnySlot {
+  int r0, rows;
+  const bf16_t *gate, *up, *down;
+};
 
-// WIDE = false handles the experts with at most 16 tokens (one chunk of token
-// rows), WIDE = true those with 17..64; both are launched and each skips the
-// other's experts.  The WIDE launch of a grouped problem is sized for the
-// most groups that can hold 17 rows (rows / 17) and its block j / nNb takes
-// the (j / nNb)-th such group.  A workgroup owns 64 consecutive weight rows (16 per wave)
-// of one expert.  GATEUP: each wave streams its 16 gate rows over all of K,
-// then the same 16 up rows, and applies SwiGLU in registers (a lane holds the
-// gate and up values of the same outputs), so at any time a workgroup reads
-// one contiguous 64-row block of one matrix: measured on the config-4 shape,
-// that streams at 6.1 TB/s where reading 32 gate and 32 up rows at once
-// reached 5.2.  The token loads of a k-chunk are issued as one group before
-// its MFMAs, so they overlap each other instead of one L2 latency per MFMA.
-template <bool GATEUP, bool WIDE>
-__global__ __launch_bounds__(256) void k_skinny_fwd(const bf16_t* __restrict__ X,
-                                                    const int* __restrict__ xrow, int kdiv,
-                                                    int xrows,
-                                                    const int* __restrict__ offsets, int ngroups,
-                                                    int Mdense,
-                                                    const bf16_t* const* w0_tab, const bf16_t* w0_one,
-                                                    const bf16_t* const* w1_tab, const bf16_t* w1_one,
-                                                    int K, int N, bf16_t* __restrict__ out0,
-                                                    bf16_t* __restrict__ out1,
-                                                    bf16_t* __restrict__ out2) {
-  constexpr int ROWS_PER_WG = kSkinnyRows;
-  constexpr int NC = WIDE ? 4 : 1;
-  constexpr int NM = GATEUP ? 2 : 1;  // weight matrices streamed in turn
-  const int nNb = (N + ROWS_PER_WG - 1) / ROWS_PER_WG;
-  const int slot = uni(blockIdx.x / nNb), nb = uni(blockIdx.x % nNb);
-  const int e = WIDE && offsets ? nth_wide_group(offsets, ngroups, slot) : slot;
-  if (e < 0) return;
-  const int r0 = offsets ? offsets[e] : 0;
-  const int M = offsets ? offsets[e + 1] - r0 : Mdense;
-  if (M <= 0 || (WIDE ? M <= 16 : M > 16)) return;
+// A skinny workgroup of NW waves: KS waves share the 16 weight rows of one row
+// block and take every KS-th k-chunk of it (partial sums added in wave order),
+// so a workgroup covers NW / KS row blocks.  The split depends on the kernel
+// alone: a token's result is the same bits in any small batch.
+//
+// What bounds it is the weights' stream, and with few experts the number of
+// bytes in flight.  Splitting K over the four waves of a workgroup instead of
+// giving each wave 16 rows of its own makes four times as many workgroups, each
+// reading 2 KB runs of a row; with gate and up rows of a chunk requested
+// together (16 loads in flight per wave, the token rows read once for both),
+// measured alone (gate/up launch): one token, six experts of 1408 x 2048 40.1
+// -> 18.6 us (3.7 TB/s); 8 tokens 88.5 -> 70.8 us (5.7 TB/s); 64 tokens, 125
+// experts of 1536 x 4096 534 -> 500 us (6.3 TB/s).  The down projection (one
+// matrix, 8 loads in flight) streams fastest with two waves to a row block:
+// 16.4 -> 9.5, 38.6 -> 33.9 and 276 -> 258 us (four waves 8.1, 34.7 and 277;
+// eight 10.7, 42.9 and 389).  Requesting the next chunk ahead of the MFMAs was
+// slower everywhere.
+constexpr int kSkinnyKsGateUp = 4, kSkinnyKsDown = 2;
+
+// LDS of the partial sums (f32x4 each).
+template <bool GATEUP, int NC, int KS, int NW>
+constexpr int skinny_red() { return (KS - 1) * (NW / KS) * (GATEUP ? 2 : 1) * NC * 64; }
+
+// Row block nb * (NW / KS) + wave / KS of W0 (and W1) against the M <= 16 NC
+// token rows r0 .. of an expert: row i is row r0 + i of X, or (xrow not null)
+// row xrow[r0 + i] / kdiv of the xrows rows of X (the assignment's token: no
+// gathered copy).  Every wave of the workgroup must call it.
+template <bool GATEUP, int NC, int KS, int NW>
+MOE_DEV void skinny_rows(f32x4* red, int nb, int r0, int M, const bf16_t* w0, const bf16_t* w1,
+                         const bf16_t* __restrict__ X, const int* __restrict__ xrow, int kdiv,
+                         int xrows, int K, int N, bf16_t* __restrict__ out0,
+                         bf16_t* __restrict__ out1, bf16_t* __restrict__ out2) {
+  constexpr int RB = NW / KS;
+  constexpr int NM = GATEUP ? 2 : 1;
   const int wave = uni(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int n0 = nb * ROWS_PER_WG + wave * 16;
+  const int rb = wave / KS, ks = wave % KS;
+  const int n0 = (nb * RB + rb) * 16;
   const int nrows = uni(min(16, N - n0));
-  if (nrows <= 0) return;  // wave-uniform; no barrier follows
   const int g = lane >> 4, rl = lane & 15;
-  // token row i of the group: row r0 + i of X, or (xrow != null) row
-  // xrow[r0 + i] / kdiv of X (the assignment's token: no gathered copy)
-  const rsrc_t rx = xrow ? make_rsrc(uni_ptr(X), (uint32_t)uni(xrows * K * 2))
-                         : make_rsrc(uni_ptr(X + (int64_t)r0 * K), (uint32_t)uni(M * K * 2));
   const int nch = (M + 15) / 16;
-  const uint32_t vw = (uint32_t)((rl * K + 8 * g) * 2);
-  uint32_t vxc[NC];
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const int i = c * 16 + rl;
-    const int row = i >= M ? -1 : xrow ? xrow[r0 + i] / kdiv : i;
-    vxc[c] = row < 0 ? kOobOffset : (uint32_t)((row * K + 8 * g) * 2);
-  }
   f32x4 acc[NM][NC];
 #pragma unroll
-  for (int m = 0; m < NM; ++m) {
+  for (int m = 0; m < NM; ++m)
 #pragma unroll
     for (int c = 0; c < NC; ++c) acc[m][c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const bf16_t* wsrc = m ? pick(w1_tab, w1_one, e) : pick(w0_tab, w0_one, e);
-    const rsrc_t rw = make_rsrc(uni_ptr(wsrc + (int64_t)n0 * K), (uint32_t)uni(nrows * K * 2));
-    for (int kc = 0; kc * 256 < K; ++kc) {
-      const uint32_t soff = (uint32_t)kc * 512;
-      u32x4 wa[8];
+  if (nrows > 0) {  // wave-uniform
+    const rsrc_t rx = xrow ? make_rsrc(uni_ptr(X), (uint32_t)uni(xrows * K * 2))
+                           : make_rsrc(uni_ptr(X + (int64_t)r0 * K), (uint32_t)uni(M * K * 2));
+    rsrc_t rw[NM];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const bool kin = kc * 256 + 32 * q + 8 * g < K;
-        wa[q] = buf_ld16(rw, kin ? vw + 64 * q : kOobOffset, soff);
-      }
+    for (int m = 0; m < NM; ++m)
+      rw[m] = make_rsrc(uni_ptr((m ? w1 : w0) + (int64_t)n0 * K), (uint32_t)uni(nrows * K * 2));
+    const uint32_t vw = (uint32_t)((rl * K + 8 * g) * 2);
+    uint32_t vxc[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int i = c * 16 + rl;
+      const int row = i >= M ? -1 : xrow ? xrow[r0 + i] / kdiv : i;
+      vxc[c] = row < 0 ? kOobOffset : (uint32_t)((row * K + 8 * g) * 2);
+    }
+    for (int kc = ks; kc * 256 < K; kc += KS) {
+      const uint32_t soff = (uint32_t)kc * 512;
+      u32x4 wa[NM][8];
+#pragma unroll
+      for (int m = 0; m < NM; ++m)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const bool kin = kc * 256 + 32 * q + 8 * g < K;
+          wa[m][q] = buf_ld16(rw[m], kin ? vw + 64 * q : kOobOffset, soff);
+        }
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
         if (c >= nch) break;
@@ -2260,9 +2186,29 @@ __global__ __launch_bounds__(256) void k_skinny_fwd(const bf16_t* __restrict__ X
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) mfma16(acc[m][c], xa[q], wa[q]);
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+          for (int q = 0; q < 8; ++q) mfma16(acc[m][c], xa[q], wa[m][q]);
       }
     }
+  }
+  if constexpr (KS > 1) {
+    if (ks > 0) {
+#pragma unroll
+      for (int m = 0; m < NM; ++m)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+          if (c < nch) red[(((ks - 1) * RB + rb) * NM * NC + m * NC + c) * 64 + lane] = acc[m][c];
+    }
+    __syncthreads();
+    if (ks > 0) return;
+#pragma unroll
+    for (int q = 1; q < KS; ++q)
+#pragma unroll
+      for (int m = 0; m < NM; ++m)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+          if (c < nch) acc[m][c] += red[(((q - 1) * RB + rb) * NM * NC + m * NC + c) * 64 + lane];
   }
   // lane holds D[token = 16 c + 4 g + r][row = rl]
   if (rl >= nrows) return;
@@ -2289,19 +2235,58 @@ __global__ __launch_bounds__(256) void k_skinny_fwd(const bf16_t* __restrict__ X
   }
 }
 
-// Router logits with few experts or few tokens (bf16): a workgroup owns 16
-// experts and 16 tokens; its kRouterWaves waves take every kRouterWaves-th
-// 256-wide k-chunk of the hidden dimension (same lane layout as k_skinny_fwd)
-// and the partial sums are added through LDS in wave order.  With few experts
-// the launch is small, so the work is cut finely (H = 4096: one chunk per
-// wave, 16 token rows per workgroup): one CU cannot pull the whole token
-// matrix quickly.
-__global__ __launch_bounds__(64 * kRouterWaves) void k_router_small(const bf16_t* __restrict__ x,
-                                                      const bf16_t* __restrict__ wr,
-                                                      const float* __restrict__ bias,
-                                                      float* __restrict__ logits, int Tn, int H,
-                                                      int E) {
-  __shared__ f32x4 red[kRouterWaves][64];
+// Routed experts (slots: blocks slot by slot, ceil(N / rows of a workgroup)
+// each) or, with slots == nullptr, the dense matrices w0, w1 over M rows of X.
+// NC: 1 for batches of at most 16 tokens, else 4.
+template <bool GATEUP, int NC, int KS>
+__global__ __launch_bounds__(256) void k_skinny_fwd(const bf16_t* __restrict__ X,
+                                                    const int* __restrict__ xrow, int kdiv,
+                                                    int xrows, const SkinnySlot* __restrict__ slots,
+                                                    int M, const bf16_t* w0, const bf16_t* w1,
+                                                    int K, int N, bf16_t* __restrict__ out0,
+                                                    bf16_t* __restrict__ out1,
+                                                    bf16_t* __restrict__ out2) {
+  __shared__ f32x4 red[skinny_red<GATEUP, NC, KS, 4>()];
+  const int nNb = (N + 16 * (4 / KS) - 1) / (16 * (4 / KS));
+  const int slot = uni(blockIdx.x / nNb), nb = uni(blockIdx.x % nNb);
+  int r0 = 0;
+  if (slots) {
+    const SkinnySlot sl = slots[slot];
+    r0 = sl.r0;
+    M = sl.rows;
+    w0 = GATEUP ? sl.gate : sl.down;
+    w1 = sl.up;
+  }
+  if (M <= 0) return;  // workgroup-uniform
+  skinny_rows<GATEUP, NC, KS, 4>(red, nb, uni(r0), uni(M), w0, w1, X, xrow, kdiv, xrows, K, N,
+                                 out0, out1, out2);
+}
+// Blocks of a launch over ng slots (or one dense problem).
+template <int KS>
+inline int skinny_grid(int ng, int N) { return ng * ((N + 16 * (4 / KS) - 1) / (16 * (4 / KS))); }
+
+// First launch of a small batch: the router logits (blocks below nrouter) and
+// the shared expert's gate/up (the blocks after them), which needs only x.
+// Router: a workgroup owns 16 experts and 16 tokens.  The hidden dimension is
+// cut into 256-wide k-chunks (same lane layout as skinny_rows); partial sum p
+// < kRouterWaves holds every kRouterWaves-th chunk, wave w computes partials w
+// and w + 8, and the partials are added through LDS in order.  With few
+// experts the router is small, so the work is cut finely: one CU cannot pull
+// the whole token matrix quickly.
+constexpr int kFrontWaves = 8;
+template <int NC>
+__global__ __launch_bounds__(64 * kFrontWaves) void k_small_front(
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ wr, const float* __restrict__ bias,
+    float* __restrict__ logits, int Tn, int H, int E, int nrouter, const bf16_t* sg,
+    const bf16_t* su, int S, bf16_t* __restrict__ sG, bf16_t* __restrict__ sU,
+    bf16_t* __restrict__ sA) {
+  constexpr int NR = skinny_red<true, NC, kFrontWaves, kFrontWaves>();
+  __shared__ f32x4 red[NR > kRouterWaves * 64 ? NR : kRouterWaves * 64];
+  if ((int)blockIdx.x >= nrouter) {
+    skinny_rows<true, NC, kFrontWaves, kFrontWaves>(red, (int)blockIdx.x - nrouter, 0, Tn, sg, su,
+                                                    x, nullptr, 1, 0, H, S, sG, sU, sA);
+    return;
+  }
   const int neb = (E + 15) / 16;
   const int e0 = uni(blockIdx.x % neb) * 16, t0 = uni(blockIdx.x / neb) * 16;
   const int wave = uni(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -2310,32 +2295,236 @@ __global__ __launch_bounds__(64 * kRouterWaves) void k_router_small(const bf16_t
   const rsrc_t rw = make_rsrc(wr + (int64_t)e0 * H, (uint32_t)((int64_t)nrows * H * 2));
   const rsrc_t rx = make_rsrc(x + (int64_t)t0 * H, (uint32_t)((int64_t)ntok * H * 2));
   const uint32_t vw = (uint32_t)((rl * H + 8 * g) * 2);
-  f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int kc = wave; kc * 256 < H; kc += kRouterWaves) {
-    const uint32_t soff = (uint32_t)kc * 512;
-    u32x4 wa[8], xa[8];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const bool kin = kc * 256 + 32 * q + 8 * g < H;
-      wa[q] = buf_ld16(rw, kin ? vw + 64 * q : kOobOffset, soff);
-      xa[q] = buf_ld16(rx, kin ? vw + 64 * q : kOobOffset, soff);
+  for (int h = 0; h < kRouterWaves / kFrontWaves; ++h) {
+    const int part = wave + h * kFrontWaves;
+    f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int kc = part; kc * 256 < H; kc += kRouterWaves) {
+      const uint32_t soff = (uint32_t)kc * 512;
+      u32x4 wa[8], xa[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const bool kin = kc * 256 + 32 * q + 8 * g < H;
+        wa[q] = buf_ld16(rw, kin ? vw + 64 * q : kOobOffset, soff);
+        xa[q] = buf_ld16(rx, kin ? vw + 64 * q : kOobOffset, soff);
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) mfma16(acc, xa[q], wa[q]);
     }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) mfma16(acc, xa[q], wa[q]);
+    red[part * 64 + lane] = acc;
   }
-  red[wave][lane] = acc;
   __syncthreads();
   if (wave != 0 || rl >= nrows) return;
   const int e = e0 + rl;
   const float b = bias ? bias[e] : 0.0f;
-  f32x4 v = red[0][lane];
+  f32x4 v = red[lane];
 #pragma unroll
-  for (int w = 1; w < kRouterWaves; ++w) v += red[w][lane];
+  for (int w = 1; w < kRouterWaves; ++w) v += red[w * 64 + lane];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int t = 4 * g + r;  // lane holds D[token t0 + 4 g + r][expert e0 + rl]
     if (t < ntok) logits[(int64_t)(t0 + t) * E + e] = v[r] + b;
   }
+}
+
+// Everything the routing of T <= kRouteSmallTokens tokens produces, in
+// workgroup 0 (16 waves): the softmax and top-k of each token (route_row, a
+// wave per token), then, from a 64-bit token mask per expert (LDS atomic ORs,
+// which do not depend on order), the counts, offsets, tile prefixes, the
+// permutation (an assignment's rank within its expert is the number of earlier
+// tokens in the mask) and the list of touched experts (`slots`, nslots of
+// them, when not null); the mean probabilities in k_colsum_partial's and
+// k_colsum_final's order (four running sums over t mod 4, added in order);
+// and, when aux or z is not null, the losses with k_losses' reduction tree.
+// No expert holds more than 64 rows, so the ten prefix sums follow from three
+// (rows, touched experts, experts of more than 32 rows), which share one
+// 32-bit scan: at most 1024 rows, 1024 experts and 31 of those (11 + 11 + 5
+// bits).  One launch instead of three (k_route, a dispatch, k_losses), whose
+// probabilities, indices and log-sum-exps stay in LDS.
+//
+// The other blocks run the shared expert's down projection beside it (its
+// gate/up ran beside the router GEMM, k_small_front), 16 waves each: it is
+// done when the routed experts start, on the call's own stream, where a side
+// stream cost two event waits of about 6 us.
+constexpr int kSmallRouteProbs = 8192;  // probabilities kept in LDS (else re-read)
+template <int EPL, int NC>
+__global__ __launch_bounds__(1024) void k_small_route(
+    const float* __restrict__ logits, int Tn, int E, int k, float tau, int norm, float c_sw,
+    float c_sq, float* __restrict__ probs, float* __restrict__ lse, int* __restrict__ idx,
+    float* __restrict__ w, float* __restrict__ P, int* __restrict__ counts,
+    int* __restrict__ offsets, int* __restrict__ tile_prefix, int* __restrict__ perm,
+    int* __restrict__ inv_perm, float* __restrict__ aux, float* __restrict__ z,
+    const bf16_t* const* gate_tab, const bf16_t* const* up_tab, const bf16_t* const* down_tab,
+    SkinnySlot* __restrict__ slots, int nslots, const bf16_t* __restrict__ sA, const bf16_t* sd,
+    int S, int H, bf16_t* __restrict__ sY) {
+  static_assert(kF32RowTile == 64, "the tile prefixes of up to 64 rows");
+  constexpr int NR = skinny_red<false, NC, 16, 16>();
+  __shared__ union U {
+    f32x4 red[NR];
+    struct {
+      float probs[kSmallRouteProbs];
+      unsigned tmask[1024][2];
+      int sidx[kRouteSmallTokens * 16];
+      int offs[1024];
+      float P[1024];
+      float lse[kRouteSmallTokens];
+      int wsum[16];
+      float r[3][256];
+    } s;
+  } u;
+  if (blockIdx.x > 0) {
+    skinny_rows<false, NC, 16, 16>(u.red, (int)blockIdx.x - 1, 0, Tn, sd, nullptr, sA, nullptr, 1,
+                                   0, S, H, sY, nullptr, nullptr);
+    return;
+  }
+  const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+  for (int e = tid; e < E; e += 1024) u.s.tmask[e][0] = u.s.tmask[e][1] = 0u;
+  __syncthreads();
+  const bool keep = Tn * E <= kSmallRouteProbs;
+  for (int t = wave; t < Tn; t += 16) {
+    float pr[EPL], l;
+    int sel;
+    route_row<EPL>(logits + (int64_t)t * E, t, E, k, tau, norm, probs, lse, idx, w, pr, sel, l);
+    if (keep) {
+#pragma unroll
+      for (int i = 0; i < EPL; ++i)
+        if (lane + 64 * i < E) u.s.probs[t * E + lane + 64 * i] = pr[i];
+    }
+    if (lane == 0) u.s.lse[t] = l;
+    if (lane < k) {
+      u.s.sidx[t * k + lane] = sel;
+      atomicOr(&u.s.tmask[sel][t >> 5], 1u << (t & 31));
+    }
+  }
+  __syncthreads();
+  // counts and the packed prefix sum, one expert per thread
+  const int c = tid < E ? __popc(u.s.tmask[tid][0]) + __popc(u.s.tmask[tid][1]) : 0;
+  const int touched = c > 0 ? 1 : 0, big = c > 32 ? 1 : 0;
+  const int mine = c | (touched << 11) | (big << 22);
+  int incl[1] = {mine};
+  wave_incl_scans(incl);
+  if (lane == 63) u.s.wsum[wave] = incl[0];
+  __syncthreads();
+  int base = 0, total = 0;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int q = u.s.wsum[v];
+    base += v < wave ? q : 0;
+    total += q;
+  }
+  {
+    const bool last = tid == E;  // writes the totals (E <= 1023; else thread 1023 does)
+    const int ex = last ? total : base + incl[0] - mine;
+    auto put = [&](int at, int q) {
+      const int off = q & 2047, tch = (q >> 11) & 2047, bg = q >> 22;
+      offsets[at] = off;
+      // [height][all, big, half]: 64-row tiles, then the two taller heights,
+      // whose only tile is a half tile
+      const int v[kTilePrefixes * kNumTileBM] = {tch, bg, tch - bg, tch, 0, tch, tch, 0, tch};
+#pragma unroll
+      for (int j = 0; j < kTilePrefixes * kNumTileBM; ++j) tile_prefix[j * (E + 1) + at] = v[j];
+    };
+    if (tid <= E) put(tid, ex);
+    if (E == 1024 && tid == 1023) put(1024, total);
+    if (tid < E) {
+      counts[tid] = c;
+      u.s.offs[tid] = ex & 2047;
+      if (slots && c > 0) {
+        const int j = (ex >> 11) & 2047;
+        if (j < nslots)
+          slots[j] = SkinnySlot{ex & 2047, c, gate_tab[tid], up_tab[tid], down_tab[tid]};
+      }
+    }
+    if (slots && tid < nslots && tid >= ((total >> 11) & 2047))
+      slots[tid] = SkinnySlot{0, 0, nullptr, nullptr, nullptr};
+  }
+  // P: lanes 4e + q hold the running sum over tokens t = q mod 4
+  const float scale = 1.0f / (float)Tn;
+  for (int e0 = 0; e0 < E; e0 += 256) {
+    const int e = e0 + (tid >> 2), q = tid & 3;
+    float r = 0.0f;
+    if (e < E) {
+      float v[kRouteSmallTokens / 4];
+#pragma unroll
+      for (int i = 0; i < kRouteSmallTokens / 4; ++i) {
+        const int t = q + 4 * i;
+        v[i] = t < Tn ? (keep ? u.s.probs[t * E + e] : probs[(int64_t)t * E + e]) : 0.0f;
+      }
+#pragma unroll
+      for (int i = 0; i < kRouteSmallTokens / 4; ++i)
+        if (q + 4 * i < Tn) r += v[i];
+    }
+    const int first = lane & 60;  // lanes 4e .. 4e + 3 of this wave
+    const float r0 = __shfl(r, first, 64), r1 = __shfl(r, first + 1, 64);
+    const float r2 = __shfl(r, first + 2, 64), r3 = __shfl(r, first + 3, 64);
+    // k_colsum_final adds this single partial to three zeros: the same value
+    if (e < E && q == 0) {
+      const float p = (((r0 + r1) + r2) + r3) * scale;
+      P[e] = p;
+      u.s.P[e] = p;
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < Tn * k; i += 1024) {
+    const int t = i / k, e = u.s.sidx[i];
+    const unsigned lo = u.s.tmask[e][0], hi = u.s.tmask[e][1];
+    const int rank = t < 32 ? __popc(lo & ((1u << t) - 1u))
+                            : __popc(lo) + __popc(hi & ((1u << (t - 32)) - 1u));
+    const int pos = u.s.offs[e] + rank;
+    perm[pos] = i;
+    inv_perm[i] = pos;
+  }
+  if (!aux && !z) return;
+  if (tid < 256) {
+    const float inv_tk = 1.0f / ((float)Tn * (float)k);
+    float sw = 0.0f, sq = 0.0f;
+    for (int e = tid; e < E; e += 256) {
+      const float p = u.s.P[e];
+      const int ce = __popc(u.s.tmask[e][0]) + __popc(u.s.tmask[e][1]);
+      sw += ((float)ce * inv_tk) * p;
+      sq += p * p;
+    }
+    u.s.r[0][tid] = sw;
+    u.s.r[1][tid] = sq;
+    u.s.r[2][tid] = tid < Tn ? u.s.lse[tid] * u.s.lse[tid] : 0.0f;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    float v[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const float* r = u.s.r[j];
+      v[j] = wave_sum((r[lane] + r[lane + 128]) + (r[lane + 64] + r[lane + 192]));
+    }
+    if (lane == 0) {
+      if (aux) *aux = (float)E * (c_sw * v[0] + c_sq * v[1]);
+      if (z) *z = v[2] / (float)Tn;
+    }
+  }
+}
+
+// The list of touched experts alone, from the kept offsets (a recomputing
+// backward, whose forward's list is gone): one block of 1024 threads.
+__global__ __launch_bounds__(1024) void k_small_slots(const int* __restrict__ offsets, int E,
+                                                      const bf16_t* const* gate_tab,
+                                                      const bf16_t* const* up_tab,
+                                                      const bf16_t* const* down_tab,
+                                                      SkinnySlot* __restrict__ slots, int nslots) {
+  __shared__ int wsum[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r0 = tid < E ? offsets[tid] : 0;
+  const int c = tid < E ? offsets[tid + 1] - r0 : 0;
+  const uint64_t m = __ballot(c > 0);
+  if (lane == 0) wsum[wave] = __popcll(m);
+  __syncthreads();
+  int base = 0, total = 0;
+  for (int v = 0; v < 16; ++v) {
+    base += v < wave ? wsum[v] : 0;
+    total += wsum[v];
+  }
+  const int j = base + __popcll(m & ((1ull << lane) - 1ull));
+  if (c > 0 && j < nslots) slots[j] = SkinnySlot{r0, c, gate_tab[tid], up_tab[tid], down_tab[tid]};
+  if (tid < nslots && tid >= total) slots[tid] = SkinnySlot{0, 0, nullptr, nullptr, nullptr};
 }
 
 }  // namespace moe

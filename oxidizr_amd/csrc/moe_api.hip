@@ -92,8 +92,8 @@ int elt_size(int dtype) { return dtype == MOE_DTYPE_F32 ? 4 : 2; }
 // The fused router kernel (router GEMM + routing + the 16-token groups'
 // histograms and probability sums) applies to plans (bf16 or fp32) with up to
 // kFusedRouterMaxExperts experts and more than kRouteSmallTokens tokens (the
-// small-token path keeps k_router_small, whose 16 x 16 blocks spread a few
-// tokens over more workgroups).  With more experts a workgroup that owns every
+// small-token path has k_small_front, whose 16 x 16 blocks spread a few tokens
+// over more workgroups).  With more experts a workgroup that owns every
 // expert of its tokens re-reads the whole router weight per 16 tokens; there
 // the tiled router GEMM and k_route stay separate.  fp32 (config 1: T = 1024,
 // H = 384, E = 8): router, route and dispatch stages 19 + 8 + 15 us fused,
@@ -109,16 +109,11 @@ bool fused_router(const moe_config& c, int64_t T) {
 int router_splits(const moe_config& c) {
   return c.hidden >= 3584 ? std::min(8, c.hidden / 1792) : 1;
 }
-// Which router GEMM a forward over T tokens runs.  The router GEMM has N = E:
-// up to kRouterSmallMaxExperts experts the 16 x 16 blocks of k_router_small
-// fill the GPU better than 128 x 128 tiles (config 2, E = 16: 31 -> 12 us; at
-// E = 64 the tiles are faster).
-constexpr int kRouterSmallMaxExperts = 32;
+// Which router GEMM a forward over T tokens runs.
 enum class RouterPath { Fused, Small, Split, Tiled };
 RouterPath router_path(const moe_config& c, int64_t T) {
   if (fused_router(c, T)) return RouterPath::Fused;
-  if (c.dtype == MOE_DTYPE_BF16 && (T <= kSkinnyMaxTokens || c.num_experts <= kRouterSmallMaxExperts))
-    return RouterPath::Small;
+  if (c.dtype == MOE_DTYPE_BF16 && T <= kSkinnyMaxTokens) return RouterPath::Small;
   return router_splits(c) > 1 ? RouterPath::Split : RouterPath::Tiled;
 }
 // The split router GEMM's partials are summed and routed by k_reduce_route
@@ -241,6 +236,9 @@ struct moe_plan {
   void* scratch_ptr = nullptr;  // device address of `scratch` on this plan's device
   // device pointer tables: 0 gate, 1 up, 2 down (weights); 3..5 their grads
   void** d_tab = nullptr;
+  // the touched experts of a small batch (bf16 plans), written by its routing
+  // and read by its expert launches; like the tables, one call at a time
+  SkinnySlot* d_slots = nullptr;
   // Pinned host staging for table uploads: a ring of kTabSlots slots of 6 E
   // pointers.  A slot is refilled only after the copy that last read it has
   // run (its event), so an upload never waits for the stream as a whole.
@@ -542,11 +540,6 @@ void launch_route(hipStream_t s, int grid, const float* logits, int T, int E, in
                      probs, lse, idx, w);
 }
 
-// Routing (from logits already in saved), losses' P statistics and dispatch.
-// pjoin != null: the mean probabilities P may be summed on the plan's
-// weight-gradient stream, forked through *pjoin; the caller joins it before
-// reading P.
-
 template <int NEB, typename D>
 void launch_router_route(hipStream_t s, int T, const D* x, const D* wr, const float* b,
                          int H, int E, int k, float tau, int norm, float* logits, float* probs,
@@ -555,15 +548,52 @@ void launch_router_route(hipStream_t s, int T, const D* x, const D* wr, const fl
                      x, wr, b, T, H, E, k, tau, norm, logits, probs, lse, idx, w, ghist, gpart);
 }
 
+// What k_small_route does beside the routing of a small batch: the losses (when
+// aux or z is not null), the list of touched experts (skinny) and the shared
+// expert's down projection sY = sA Wd^T (S > 0).
+struct SmallExtra {
+  float* aux = nullptr;
+  float* z = nullptr;
+  bool skinny = false;
+  int S = 0;
+  const bf16_t* sA = nullptr;
+  const bf16_t* sd = nullptr;
+  bf16_t* sY = nullptr;
+};
+// Touched experts of T tokens: at most one per assignment.
+int small_slots(const moe_config& c, int64_t T) {
+  return (int)std::min<int64_t>(c.num_experts, T * c.experts_per_tok);
+}
+template <int EPL, int NC, typename D>
+void launch_small_route(moe_plan* p, hipStream_t s, int T, char* saved, const SavedLayout& L,
+                        const SmallExtra& x) {
+  const moe_config& c = p->cfg;
+  const int E = c.num_experts, H = c.hidden;
+  auto f = [&](int id) { return (float*)(saved + L.f[id]); };
+  auto i = [&](int id) { return (int*)(saved + L.f[id]); };
+  const bf16_t* const* tab = (const bf16_t* const*)p->d_tab;
+  hipLaunchKernelGGL((k_small_route<EPL, NC>), dim3(1 + (x.S > 0 ? ceil_div(H, 16) : 0)),
+                     dim3(1024), 0, s, f(MOE_SAVED_LOGITS), T, E, c.experts_per_tok,
+                     c.router_temperature, c.norm_topk_prob, c.aux_switch_coef, c.aux_sqprob_coef,
+                     f(MOE_SAVED_PROBS), f(MOE_SAVED_LSE), i(MOE_SAVED_TOPK_IDX),
+                     f(MOE_SAVED_TOPK_W), f(MOE_SAVED_MEAN_PROB), i(MOE_SAVED_COUNTS),
+                     i(MOE_SAVED_OFFSETS), (int*)(saved + L.tile_prefix), i(MOE_SAVED_PERM),
+                     i(MOE_SAVED_INV_PERM), x.aux, x.z, tab, tab + E, tab + 2 * E,
+                     x.skinny ? p->d_slots : nullptr, small_slots(c, T), x.sA, x.sd, x.S, H, x.sY);
+}
+
 // Routing (from logits already in saved, unless `routed`: the fused router
 // kernel has written the routing decisions too), losses' P statistics and
 // dispatch.  With `routed` (T > kRouteSmallTokens) the dispatch stops after
 // k_scan: the caller writes perm and inv_perm (k_scatter_groups from the
-// group bases at W.gbase).
+// group bases at W.gbase).  pjoin != null: the mean probabilities P may be
+// summed on the plan's weight-gradient stream, forked through *pjoin; the
+// caller joins it before reading P.  Up to kRouteSmallTokens tokens everything
+// is one launch (k_small_route, with `extra`).
 template <typename D>
 moe_status run_routing(moe_plan* p, hipStream_t s, int64_t T64, char* saved, char* ws,
                        const SavedLayout& L, const WsLayout& W, SideJoin* pjoin,
-                       bool routed = false) {
+                       bool routed = false, const SmallExtra& extra = {}) {
   const moe_config& c = p->cfg;
   const int T = (int)T64, E = c.num_experts, k = c.experts_per_tok;
   float* logits = (float*)(saved + L.f[MOE_SAVED_LOGITS]);
@@ -577,6 +607,22 @@ moe_status run_routing(moe_plan* p, hipStream_t s, int64_t T64, char* saved, cha
   int* inv = (int*)(saved + L.f[MOE_SAVED_INV_PERM]);
   float* P = (float*)(saved + L.f[MOE_SAVED_MEAN_PROB]);
   int* tprefix = (int*)(saved + L.tile_prefix);
+  if (T <= kRouteSmallTokens) {
+    StageTimer st(p, s, MOE_STAGE_ROUTE);
+    auto go = [&](auto epl) {
+      if (T <= 16) launch_small_route<decltype(epl)::value, 1, D>(p, s, T, saved, L, extra);
+      else launch_small_route<decltype(epl)::value, 4, D>(p, s, T, saved, L, extra);
+    };
+    switch (route_epl(E)) {
+      case 1: go(std::integral_constant<int, 1>()); break;
+      case 2: go(std::integral_constant<int, 2>()); break;
+      case 4: go(std::integral_constant<int, 4>()); break;
+      case 8: go(std::integral_constant<int, 8>()); break;
+      default: go(std::integral_constant<int, 16>()); break;
+    }
+    LAUNCH_CHECK();
+    return MOE_OK;
+  }
   {
     StageTimer st(p, s, MOE_STAGE_ROUTE);
     const int grid = ceil_div(T, 4);
@@ -589,12 +635,6 @@ moe_status run_routing(moe_plan* p, hipStream_t s, int64_t T64, char* saved, cha
       default: launch_route<16>(s, grid, logits, T, E, k, tau, c.norm_topk_prob, probs, lse, idx, w); break;
     }
     LAUNCH_CHECK();
-    if (T <= kRouteSmallTokens) {  // P and the whole dispatch in one workgroup
-      hipLaunchKernelGGL(k_dispatch_small, dim3(1), dim3(1024), 0, s, idx, probs, T, E, k,
-                         1.0f / (float)T, P, counts, offsets, tprefix, perm, inv);
-      LAUNCH_CHECK();
-      return MOE_OK;
-    }
     const hipStream_t ps = pjoin ? p->wgrad_stream(s) : s;
     if (pjoin) HIP_TRY(pjoin->fork(s, ps, p->wfork, p->wjoin));
     if (routed) {  // P from the fused router's per-group sums, in two fixed-order levels
@@ -740,25 +780,17 @@ void shared_fwd(moe_plan* p, hipStream_t ss, int T, const D* x, const moe_weight
   using CG = typename Tilings<D>::GateUp;
   using CB = typename Tilings<D>::Big;
   const int H = p->cfg.hidden, S = p->cfg.shared_intermediate;
-  const bool skinny = std::is_same<D, bf16_t>::value && T <= kSkinnyMaxTokens;
-  if (skinny && T <= 16) {
-    hipLaunchKernelGGL((k_skinny_fwd<true, false>), dim3(ceil_div(S, kSkinnyRows)), dim3(256), kSkinnyLdsReserve, ss,
-                       (const bf16_t*)x, nullptr, 1, 0, nullptr, 1, T, nullptr, (const bf16_t*)w->shared_gate,
-                       nullptr, (const bf16_t*)w->shared_up, H, S, (bf16_t*)sG, (bf16_t*)sU,
-                       (bf16_t*)sA);
-    if (sY)
-      hipLaunchKernelGGL((k_skinny_fwd<false, false>), dim3(ceil_div(H, kSkinnyRows)), dim3(256), kSkinnyLdsReserve, ss,
-                         (const bf16_t*)sA, nullptr, 1, 0, nullptr, 1, T, nullptr, (const bf16_t*)w->shared_down,
-                         nullptr, nullptr, S, H, (bf16_t*)sY, nullptr, nullptr);
-  } else if (skinny) {
-    hipLaunchKernelGGL((k_skinny_fwd<true, true>), dim3(ceil_div(S, kSkinnyRows)), dim3(256), 0, ss,
-                       (const bf16_t*)x, nullptr, 1, 0, nullptr, 1, T, nullptr, (const bf16_t*)w->shared_gate,
-                       nullptr, (const bf16_t*)w->shared_up, H, S, (bf16_t*)sG, (bf16_t*)sU,
-                       (bf16_t*)sA);
-    if (sY)
-      hipLaunchKernelGGL((k_skinny_fwd<false, true>), dim3(ceil_div(H, kSkinnyRows)), dim3(256), 0, ss,
-                         (const bf16_t*)sA, nullptr, 1, 0, nullptr, 1, T, nullptr, (const bf16_t*)w->shared_down,
-                         nullptr, nullptr, S, H, (bf16_t*)sY, nullptr, nullptr);
+  if (std::is_same<D, bf16_t>::value && T <= kSkinnyMaxTokens) {
+    // a recomputing backward's activations, which need no down projection: the
+    // shared part of the forward's launch
+    auto go = [&](auto nc) {
+      hipLaunchKernelGGL((k_small_front<decltype(nc)::value>), dim3(ceil_div(S, 16)),
+                         dim3(64 * kFrontWaves), 0, ss, (const bf16_t*)x, nullptr, nullptr, nullptr,
+                         T, H, p->cfg.num_experts, 0, (const bf16_t*)w->shared_gate,
+                         (const bf16_t*)w->shared_up, S, (bf16_t*)sG, (bf16_t*)sU, (bf16_t*)sA);
+    };
+    if (T <= 16) go(std::integral_constant<int, 1>());
+    else go(std::integral_constant<int, 4>());
   } else {
     const RowGroups dense{nullptr, nullptr, nullptr, nullptr, 1, T, 0, 0};
     with_dense_tiling<D, CG>(T, S, [&](auto c, int grid) {
@@ -838,7 +870,8 @@ moe_status routed_fwd(moe_plan* p, hipStream_t s, int T, const D* x, const State
   const int H = c.hidden, E = c.num_experts, k = c.experts_per_tok, I = c.intermediate;
   const int64_t TK = (int64_t)T * k;
   auto stage = [&](int id) { return timed ? id : MOE_STAGE_RECOMPUTE; };
-  // few tokens: no expert holds more than T rows, stream the weights instead
+  // few tokens: no expert holds more than T rows, stream the weights of the
+  // experts that the routing listed (p->d_slots) instead
   const bool skinny = std::is_same<D, bf16_t>::value && T <= kSkinnyMaxTokens;
   if (gbase) {  // the dispatch's last launch
     StageTimer tm(p, s, stage(MOE_STAGE_DISPATCH));
@@ -846,23 +879,21 @@ moe_status routed_fwd(moe_plan* p, hipStream_t s, int T, const D* x, const State
                        gbase, st.perm, st.inv);
     LAUNCH_CHECK();
   }
-  const bf16_t* xsrc = (const bf16_t*)x;
-  const int* xrow = st.perm;
   const D* const* tg = (const D* const*)p->d_tab;
   const D* const* tu = (const D* const*)(p->d_tab + E);
   const D* const* td = (const D* const*)(p->d_tab + 2 * E);
   {
     StageTimer tm(p, s, stage(MOE_STAGE_GATEUP_FWD));
     if (skinny) {
-      hipLaunchKernelGGL((k_skinny_fwd<true, false>), dim3(E * ceil_div(I, kSkinnyRows)), dim3(256), kSkinnyLdsReserve, s,
-                         xsrc, xrow, k, T, st.offsets, E, 0, (const bf16_t* const*)tg, nullptr,
-                         (const bf16_t* const*)tu, nullptr, H, I, (bf16_t*)st.G, (bf16_t*)st.U,
-                         (bf16_t*)st.A);
-      if (T > 16)
-        hipLaunchKernelGGL((k_skinny_fwd<true, true>), dim3(max_wide_groups(TK, E) * ceil_div(I, kSkinnyRows)), dim3(256), 0, s,
-                           xsrc, xrow, k, T, st.offsets, E, 0, (const bf16_t* const*)tg,
-                           nullptr, (const bf16_t* const*)tu, nullptr, H, I, (bf16_t*)st.G,
-                           (bf16_t*)st.U, (bf16_t*)st.A);
+      constexpr int KS = kSkinnyKsGateUp;
+      auto go = [&](auto nc) {
+        hipLaunchKernelGGL((k_skinny_fwd<true, decltype(nc)::value, KS>),
+                           dim3(skinny_grid<KS>(small_slots(c, T), I)), dim3(256), 0, s,
+                           (const bf16_t*)x, st.perm, k, T, p->d_slots, 0, nullptr, nullptr, H, I,
+                           (bf16_t*)st.G, (bf16_t*)st.U, (bf16_t*)st.A);
+      };
+      if (T <= 16) go(std::integral_constant<int, 1>());
+      else go(std::integral_constant<int, 4>());
     } else {
       with_row_tiling<D, CG>(st.offsets, st.tprefix, E, TK, [&](auto c, const RowGroups& r, auto grid) {
         using C = decltype(c);
@@ -877,13 +908,15 @@ moe_status routed_fwd(moe_plan* p, hipStream_t s, int T, const D* x, const State
   {
     StageTimer tm(p, s, stage(MOE_STAGE_DOWN_FWD));
     if (skinny) {
-      hipLaunchKernelGGL((k_skinny_fwd<false, false>), dim3(E * ceil_div(H, kSkinnyRows)), dim3(256), kSkinnyLdsReserve, s,
-                         (const bf16_t*)st.A, nullptr, 1, 0, st.offsets, E, 0, (const bf16_t* const*)td, nullptr,
-                         nullptr, nullptr, I, H, (bf16_t*)st.Y, nullptr, nullptr);
-      if (T > 16)
-        hipLaunchKernelGGL((k_skinny_fwd<false, true>), dim3(max_wide_groups(TK, E) * ceil_div(H, kSkinnyRows)), dim3(256), 0,
-                           s, (const bf16_t*)st.A, nullptr, 1, 0, st.offsets, E, 0, (const bf16_t* const*)td,
-                           nullptr, nullptr, nullptr, I, H, (bf16_t*)st.Y, nullptr, nullptr);
+      constexpr int KS = kSkinnyKsDown;
+      auto go = [&](auto nc) {
+        hipLaunchKernelGGL((k_skinny_fwd<false, decltype(nc)::value, KS>),
+                           dim3(skinny_grid<KS>(small_slots(c, T), H)), dim3(256), 0, s,
+                           (const bf16_t*)st.A, nullptr, 1, 0, p->d_slots, 0, nullptr, nullptr, I,
+                           H, (bf16_t*)st.Y, nullptr, nullptr);
+      };
+      if (T <= 16) go(std::integral_constant<int, 1>());
+      else go(std::integral_constant<int, 4>());
     } else {
       with_row_tiling<D, CB>(st.offsets, st.tprefix, E, TK, [&](auto c, const RowGroups& r, auto grid) {
         using C = decltype(c);
@@ -923,14 +956,15 @@ moe_status forward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* x,
   // a kept training forward still needs the expert outputs for its combine:
   // they go to the forward-only region, unused by such a call
   if (!st.Y) st.Y = (D*)(ws + W.infer + LT.f[MOE_SAVED_EXPERT_OUT]);
-  // Shared expert first, on the plan's second stream: it only needs x.
-  D* sY = nullptr;
+  // Shared expert first, on the plan's second stream: it only needs x.  A
+  // small bf16 batch runs it beside the router on the call's own stream.
+  const bool skinny = std::is_same<D, bf16_t>::value && T <= kSkinnyMaxTokens;
+  D* sY = S > 0 ? (D*)(ws + W.sY) : nullptr;
   SideJoin shared_join, p_join;
-  if (S > 0) {
+  if (S > 0 && !skinny) {
     const hipStream_t ss = p->shared_stream(s);
     HIP_TRY(shared_join.fork(s, ss, p->fork, p->join));
     StageTimer tm(p, ss, MOE_STAGE_SHARED_FWD);
-    sY = (D*)(ws + W.sY);
     shared_fwd<D>(p, ss, T, x, w, st.sG, st.sU, st.sA, sY);
     LAUNCH_CHECK();
   }
@@ -953,10 +987,17 @@ moe_status forward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* x,
       else
         launch_router_route<4, D>(s, T, xb, wrb, rbias, H, E, k, tau, nt, st.logits, st.probs, st.lse, st.idx, st.w, gh, gp);
     } else if (rp == RouterPath::Small) {
-      hipLaunchKernelGGL(k_router_small, dim3(ceil_div(E, 16) * ceil_div(T, 16)),
-                         dim3(64 * kRouterWaves), 0, s, (const bf16_t*)x,
-                         (const bf16_t*)w->router, c.has_router_bias ? w->router_bias : nullptr,
-                         st.logits, T, H, E);
+      const int nr = ceil_div(E, 16) * ceil_div(T, 16);
+      auto go = [&](auto nc) {
+        hipLaunchKernelGGL((k_small_front<decltype(nc)::value>),
+                           dim3(nr + (S > 0 ? ceil_div(S, 16) : 0)), dim3(64 * kFrontWaves),
+                           0, s, (const bf16_t*)x, (const bf16_t*)w->router,
+                           c.has_router_bias ? w->router_bias : nullptr, st.logits, T, H, E, nr,
+                           (const bf16_t*)w->shared_gate, (const bf16_t*)w->shared_up, S,
+                           (bf16_t*)st.sG, (bf16_t*)st.sU, (bf16_t*)st.sA);
+      };
+      if (T <= 16) go(std::integral_constant<int, 1>());
+      else go(std::integral_constant<int, 4>());
     } else if (rp == RouterPath::Split) {
       const int ns = router_splits(c);
       float* part = (float*)(ws + W.rpart);
@@ -1000,9 +1041,19 @@ moe_status forward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* x,
   // the fused router's dispatch stops after k_scan; the routed forward's
   // first launch (k_scatter_groups) writes perm and inv_perm
   const bool defer = fused;
-  moe_status r = run_routing<D>(p, s, T64, rb, ws, LR, W, &p_join, fused);
+  SmallExtra extra;
+  extra.aux = aux;
+  extra.z = z;
+  if (skinny) {
+    extra.skinny = true;
+    extra.S = S;
+    extra.sA = (const bf16_t*)st.sA;
+    extra.sd = (const bf16_t*)w->shared_down;
+    extra.sY = (bf16_t*)sY;
+  }
+  moe_status r = run_routing<D>(p, s, T64, rb, ws, LR, W, &p_join, fused, extra);
   if (r != MOE_OK) return r;
-  {
+  if (T > kRouteSmallTokens) {  // k_small_route forms a small batch's losses
     // beside the dispatch when P is summed on the side stream (the kernel
     // then counts the experts itself), else after the dispatch on s
     const bool side = p_join.armed;
@@ -1021,7 +1072,6 @@ moe_status forward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* x,
     const int nsl = ceil_div(H / (16 / (int)sizeof(D)), kCombineSlice);
     // the tiled down projection writes Y token-major; the small-token kernel
     // in expert order
-    const bool skinny = std::is_same<D, bf16_t>::value && T <= kSkinnyMaxTokens;
     hipLaunchKernelGGL(k_combine_fwd<D>, dim3(ceil_div((int64_t)T * nsl, 4)), dim3(256), 0, s,
                        st.Y, skinny ? st.inv : nullptr,
                        st.w, sY, c.shared_expert_scale, T, k, H, resid, out);
@@ -1141,6 +1191,12 @@ moe_status backward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* dout,
     if (rs != MOE_OK) return rs;
   }
   if (recompute) {
+    if (std::is_same<D, bf16_t>::value && T <= kSkinnyMaxTokens) {
+      const bf16_t* const* tab = (const bf16_t* const*)p->d_tab;
+      hipLaunchKernelGGL(k_small_slots, dim3(1), dim3(1024), 0, s, offsets, E, tab, tab + E,
+                         tab + 2 * E, p->d_slots, small_slots(c, T));
+      LAUNCH_CHECK();
+    }
     moe_status r = routed_fwd<D>(p, s, T, x, st, false);
     if (r != MOE_OK) return r;
   }
@@ -1527,6 +1583,8 @@ moe_status moe_plan_create(const moe_config* cfg, int device, moe_plan** out) {
   if (e == hipSuccess)
     e = hipHostMalloc((void**)&p->h_tab, tab_bytes * moe_plan::kTabSlots, hipHostMallocDefault);
   if (e == hipSuccess) e = hipMemset(p->d_tab, 0, tab_bytes);
+  if (e == hipSuccess && cfg->dtype == MOE_DTYPE_BF16)
+    e = hipMalloc((void**)&p->d_slots, sizeof(SkinnySlot) * (size_t)cfg->num_experts);
   for (int i = 0; i < moe_plan::kTabSlots && e == hipSuccess; ++i)
     e = hipEventCreateWithFlags(&p->tab_ev[i], hipEventDisableTiming);
   if (e == hipSuccess && cfg->shared_intermediate > 0) {
@@ -1574,6 +1632,7 @@ moe_status moe_plan_destroy(moe_plan* p) {
     (void)hipEventDestroy(p->tab_ev[i]);
   }
   if (p->d_tab) (void)hipFree(p->d_tab);
+  if (p->d_slots) (void)hipFree(p->d_slots);
   if (p->h_tab) (void)hipHostFree(p->h_tab);
   if (p->xflag_ev) {
     if (p->xflag_pending) (void)hipEventSynchronize(p->xflag_ev);
