@@ -47,6 +47,21 @@ template <> struct Tilings<bf16_t> {
   using GateUp = Tiling<bf16_t, 256, 128, 64, 2, 2, 8>;
   using Big = Tiling<bf16_t, 256, 256, 64, 2, 2, 8>;
   using WgradPair = Tiling<bf16_t, 128, 256, 64, 2, 2, 8>;
+  // Shorter tilings of the gate/up forward and of the others for launches with
+  // few tiles (the rule is where the launches are, with_dense_tiling).
+  using GateUpMid = Tiling<bf16_t, 128, 64, 64, 2, 2, 4>;
+  using GateUpSmall = Tiling<bf16_t, 64, 64, 64, 2, 3, 4>;
+  using BigMid = Tiling<bf16_t, 128, 128, 64, 2, 2, 4>;
+  using BigSmall = Tiling<bf16_t, 64, 128, 64, 4, 3, 4>;
+};
+// The shorter tilings of a row-grouped or dense tiling C.
+template <class C>
+struct LowTilings {
+  static constexpr bool GATEUP = std::is_same<C, Tilings<bf16_t>::GateUp>::value;
+  using Mid = typename std::conditional<GATEUP, Tilings<bf16_t>::GateUpMid,
+                                        Tilings<bf16_t>::BigMid>::type;
+  using Small = typename std::conditional<GATEUP, Tilings<bf16_t>::GateUpSmall,
+                                          Tilings<bf16_t>::BigSmall>::type;
 };
 // fp32 (config 1: T = 1024, H = 384, I = 1024): 64-column tiles give the
 // N = H GEMMs 96 workgroups instead of the 48 that 128-column tiles leave for
@@ -772,15 +787,19 @@ __global__ __launch_bounds__(256) void k_hist(const int* __restrict__ idx, int T
   for (int e = threadIdx.x; e < E; e += 256) block_hist[(int64_t)blockIdx.x * E + e] = hist[e];
 }
 
-// counts, exclusive offsets, per-block bases, and GEMM tile prefixes for the
-// row-tile heights in kTileBM: per height, the prefixes of all, big and half
-// row tiles (RowGroups), each [E + 1].
-constexpr int kTilePrefixes = 3;
-constexpr int kNumTileBM = 3;
-__constant__ int kTileBM[kNumTileBM] = {kF32RowTile, 256, 384};
+// GEMM tile prefixes, each [E + 1]: of all row tiles for the four tile heights,
+// and of the big and half row tiles (RowGroups) for the heights whose launches
+// may run their half tiles last (256 and 384).
+constexpr int kNumTilePrefixes = 8;
+constexpr int kPrefixBM[kNumTilePrefixes] = {kF32RowTile, 128, 256, 256, 256, 384, 384, 384};
+constexpr int kPrefixKind[kNumTilePrefixes] = {0, 0, 0, 1, 2, 0, 1, 2};  // all, big, half
+// Index of the "all" prefix of a height; big and half follow it.
+constexpr int prefix_slot(int bm) {
+  return bm == kF32RowTile ? 0 : bm == 128 ? 1 : bm == 256 ? 2 : 5;
+}
 // Tail rows a group's last full row tile takes (RowGroups::tall) for row
-// tiles of height bm: the bf16 256-row tilings run it as a tall tile; fp32's
-// 128-row tiles take none.
+// tiles of height bm: the bf16 256-row tilings run it as a tall tile; the
+// others take none.
 constexpr int tall_rows_for(int bm) { return bm == 256 ? bm / 4 : 0; }
 
 // Inclusive prefix sums across the 64 lanes of a wave of N values at once:
@@ -801,13 +820,13 @@ MOE_DEV void wave_incl_scans(int (&v)[N]) {
 }
 
 // With cnt[e] (LDS, e < E <= 1024) in place, a block of 1024 threads writes
-// the exclusive offsets (also to offs, LDS) and the tile prefixes of every
-// height in kTileBM, one expert per thread.  The kScanCount scans run
+// the exclusive offsets (also to offs, LDS) and the tile prefixes, one expert
+// per thread.  The kScanCount scans run
 // together: a wave scan each, the wave totals to wsum[j][wave] (LDS,
 // kScanCount x 16), one barrier, and each thread adds the totals of the
 // waves below it with a fixed-trip predicated loop (its LDS reads all in
 // flight).  Integer arithmetic only.
-constexpr int kScanCount = 1 + kTilePrefixes * kNumTileBM;
+constexpr int kScanCount = 1 + kNumTilePrefixes;
 MOE_DEV void scan_counts(const int* cnt, int E, int* __restrict__ offsets,
                          int* __restrict__ tile_prefix, int* offs, int* wsum) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -817,7 +836,7 @@ MOE_DEV void scan_counts(const int* cnt, int E, int* __restrict__ offsets,
   for (int j = 0; j < kScanCount; ++j) {
     v[j] = c;
     if (j > 0) {
-      const int bm = kTileBM[(j - 1) / kTilePrefixes], r = c % bm, kind = (j - 1) % kTilePrefixes;
+      const int bm = kPrefixBM[j - 1], r = c % bm, kind = kPrefixKind[j - 1];
       // a short tail behind a full tile joins that tile (tall tile)
       const int merged = c > bm && r > 0 && r <= tall_rows_for(bm) ? 1 : 0;
       const int tail = r > 0 && !merged ? 1 : 0;
@@ -851,8 +870,8 @@ MOE_DEV void scan_counts(const int* cnt, int E, int* __restrict__ offsets,
 // owns expert e's histogram entries of a contiguous chunk of blocks: the
 // chunk sums and their exclusive prefix over g (a log-step scan in LDS) give
 // the expert counts and the chunk bases; the expert counts are then scanned
-// in parallel (one expert per thread) for the offsets and for the tile prefix
-// of every height in kTileBM; a last pass writes every block's base.  Chunks
+// in parallel (one expert per thread) for the offsets and for the tile
+// prefixes; a last pass writes every block's base.  Chunks
 // of up to kScanRegChunk blocks stay in registers between the two passes (one
 // round of loads, all in flight); longer ones are read twice, eight loads in
 // flight.  Integer arithmetic only.
@@ -2336,10 +2355,10 @@ __global__ __launch_bounds__(64 * kFrontWaves) void k_small_front(
 // them, when not null); the mean probabilities in k_colsum_partial's and
 // k_colsum_final's order (four running sums over t mod 4, added in order);
 // and, when aux or z is not null, the losses with k_losses' reduction tree.
-// No expert holds more than 64 rows, so the ten prefix sums follow from three
-// (rows, touched experts, experts of more than 32 rows), which share one
-// 32-bit scan: at most 1024 rows, 1024 experts and 31 of those (11 + 11 + 5
-// bits).  One launch instead of three (k_route, a dispatch, k_losses), whose
+// No expert holds more than 64 rows, so every tile prefix follows from the
+// number of touched experts (a touched expert is one row tile of any height, a
+// half tile where those are counted), and one 32-bit scan carries rows and
+// touched experts (at most 1024 each).  One launch instead of three (k_route, a dispatch, k_losses), whose
 // probabilities, indices and log-sum-exps stay in LDS.
 //
 // The other blocks run the shared expert's down projection beside it (its
@@ -2364,7 +2383,7 @@ __global__ __launch_bounds__(1024) void k_small_route(
     const bf16_t* const* gate_tab, const bf16_t* const* up_tab, const bf16_t* const* down_tab,
     SkinnySlot* __restrict__ slots, int nslots, const bf16_t* __restrict__ sA, const bf16_t* sd,
     int S, int H, bf16_t* __restrict__ sY) {
-  static_assert(kF32RowTile == 64, "the tile prefixes of up to 64 rows");
+  static_assert(kF32RowTile >= kRouteSmallTokens, "a touched expert is one row tile");
   constexpr int NR = skinny_red<false, NC, 16, 16>();
   __shared__ union U {
     f32x4 red[NR];
@@ -2406,8 +2425,7 @@ __global__ __launch_bounds__(1024) void k_small_route(
   __syncthreads();
   // counts and the packed prefix sum, one expert per thread
   const int c = tid < E ? __popc(u.s.tmask[tid][0]) + __popc(u.s.tmask[tid][1]) : 0;
-  const int touched = c > 0 ? 1 : 0, big = c > 32 ? 1 : 0;
-  const int mine = c | (touched << 11) | (big << 22);
+  const int mine = c | (c > 0 ? 1 << 16 : 0);
   int incl[1] = {mine};
   wave_incl_scans(incl);
   if (lane == 63) u.s.wsum[wave] = incl[0];
@@ -2423,26 +2441,23 @@ __global__ __launch_bounds__(1024) void k_small_route(
     const bool last = tid == E;  // writes the totals (E <= 1023; else thread 1023 does)
     const int ex = last ? total : base + incl[0] - mine;
     auto put = [&](int at, int q) {
-      const int off = q & 2047, tch = (q >> 11) & 2047, bg = q >> 22;
-      offsets[at] = off;
-      // [height][all, big, half]: 64-row tiles, then the two taller heights,
-      // whose only tile is a half tile
-      const int v[kTilePrefixes * kNumTileBM] = {tch, bg, tch - bg, tch, 0, tch, tch, 0, tch};
+      offsets[at] = q & 0xffff;
 #pragma unroll
-      for (int j = 0; j < kTilePrefixes * kNumTileBM; ++j) tile_prefix[j * (E + 1) + at] = v[j];
+      for (int j = 0; j < kNumTilePrefixes; ++j)
+        tile_prefix[j * (E + 1) + at] = kPrefixKind[j] == 1 ? 0 : q >> 16;
     };
     if (tid <= E) put(tid, ex);
     if (E == 1024 && tid == 1023) put(1024, total);
     if (tid < E) {
       counts[tid] = c;
-      u.s.offs[tid] = ex & 2047;
+      u.s.offs[tid] = ex & 0xffff;
       if (slots && c > 0) {
-        const int j = (ex >> 11) & 2047;
+        const int j = ex >> 16;
         if (j < nslots)
-          slots[j] = SkinnySlot{ex & 2047, c, gate_tab[tid], up_tab[tid], down_tab[tid]};
+          slots[j] = SkinnySlot{ex & 0xffff, c, gate_tab[tid], up_tab[tid], down_tab[tid]};
       }
     }
-    if (slots && tid < nslots && tid >= ((total >> 11) & 2047))
+    if (slots && tid < nslots && tid >= (total >> 16))
       slots[tid] = SkinnySlot{0, 0, nullptr, nullptr, nullptr};
   }
   // P: lanes 4e + q hold the running sum over tokens t = q mod 4

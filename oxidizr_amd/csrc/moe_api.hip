@@ -3,6 +3,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <mutex>
 #include <new>
@@ -307,7 +308,7 @@ struct moe_plan {
     fld(MOE_SAVED_PERM, 4 * TK);
     fld(MOE_SAVED_INV_PERM, 4 * TK);
     fld(MOE_SAVED_MEAN_PROB, 4 * (size_t)E);
-    L.tile_prefix = c.take(4 * (size_t)kTilePrefixes * kNumTileBM * (E + 1));
+    L.tile_prefix = c.take(4 * (size_t)kNumTilePrefixes * (E + 1));
     const bool act = keep != Keep::Routing, pre = keep == Keep::All;
     // the GEMMs read x through the permutation: no permuted copy is kept
     fld(MOE_SAVED_X_PERM, 0);
@@ -675,11 +676,6 @@ moe_status run_routing(moe_plan* p, hipStream_t s, int64_t T64, char* saved, cha
   return MOE_OK;
 }
 
-// Index of a row-tile height in kTileBM (the row-grouped tilings use 128
-// (fp32) and 256 (bf16) rows).
-constexpr int tile_slot(int bm) { return bm == kF32RowTile ? 0 : bm == 256 ? 1 : 2; }
-static_assert(kNumTileBM == 3, "tile_slot covers the heights of kTileBM");
-
 // Blocks of a K-grouped (weight-gradient) launch over `groups` groups or
 // split chunks of an M x N output: each takes 8 * ceil(tiles / 8) blocks.
 inline int kgrouped_grid(int groups, int M, int N, int BM, int BN) {
@@ -751,29 +747,115 @@ struct State {
   }
 };
 
-// Shared expert forward over all T tokens on stream ss: G, U (when kept), A,
-// and the down projection into sY when sY is not null.
-// Calls f(tiling, grid) for a dense (shared-expert) launch of tiling C over
-// T rows and N columns: C, or its 384-row tiles when those fill fewer whole
-// rounds of 256 CUs, a 384-row tile counted at kDense384Cost tenths of a
-// 256-row one (a k-tile brings 25 % more operand rows for 50 % more MFMA
-// work).  The last row tile runs as the shortest tiling that covers it.
-constexpr int kDense384Cost = 14;
-template <typename D, class C, class F>
-void with_dense_tiling(int T, int N, F&& f) {
-  const int64_t nN = ceil_div(N, C::BN);
-  if constexpr (has_half_rows<D, C>()) {
-    using C3 = Rows384<C>;
-    const int64_t r256 = ceil_div(ceil_div(T, C::BM) * nN, (int64_t)256);
-    const int64_t r384 = ceil_div(ceil_div(T, C3::AR) * nN, (int64_t)256);
-    if (kDense384Cost * r384 < 10 * r256) {
-      f(C3{}, (int)(ceil_div(T, C3::AR) * nN));
-      return;
-    }
-  }
-  f(C{}, (int)(ceil_div(T, C::BM) * nN));
+// ---- tiling of a dense or row-grouped launch
+//
+// One 256 x 256 (or 384-row) tile per CU is the fastest way through a launch
+// that fills the CUs with them.  A launch with fewer leaves CUs idle for a
+// whole tile: its time is one tile's, a serial chain of K / 64 k-tiles, however
+// few rows there are.  128 x 128 tiles (two workgroups to a CU) and 64 x 128
+// tiles (two, three stages) bring fewer bytes per k-tile and fill the CUs from
+// four or eight times fewer rows; every output keeps its k order (same bits).
+//
+// The rule compares rounds of tiles, in units of a tenth of a 256-row tile:
+// `one` for a round of up to 256 tiles (one to a CU), `two` for one of up to
+// 512.  Measured per k-tile of 64 on dense launches alone, K = 1536 .. 4096, N
+// = 1536 .. 4096, T = 128 .. 4096, against the 256-row tile (down 1.16 us,
+// gate/up 1.44, gate/up input gradient 1.43, down input gradient 1.9 with its
+// epilogue):
+//   128 x 128     one 0.6-0.72, two 0.72-0.86    (down 0.83, 1.0 us)
+//   64 x 128      one 0.31-0.48, two 0.51-0.59   (down 0.40, 0.69 us)
+//   gate/up 128 x 64: 0.5-0.55, 0.7;  64 x 64: 0.30, 0.47
+// T = 500, H = 2048, S = 2816 alone, 256-row tiles -> picked: gate/up forward 44
+// -> 22 us, down 50 -> 18, down input gradient 60 -> 27, gate/up input gradient
+// 127 -> 61.  An experts' launch counts its rows as evenly spread (an expert's
+// last tile half empty on average) and changes only for an estimated gain of 15
+// %: weights that stream from memory set the time of launches with few rows per
+// expert, whatever the tile.  Alone, 16 experts of 62 rows (H = 2048, I = 1408):
+// down input gradient 42 -> 29 us, gate/up input gradient 49 -> 38; 8 experts of
+// 500 rows (H = 1024, I = 2048): gate/up input gradient 101 -> 58.
+//
+// The shorter tilings take more CU time for the same work, so they pay only
+// while a routed launch and the shared expert's beside it leave CUs idle: below
+// kBusyTiles 256-row tiles in both, that hold fewer rows than kBusyRows full
+// ones (leaves_idle).  Steps (fwd + bwd, E = 16, k = 2, H = 2048, I = 1408, S =
+// 2816): T = 300 481 -> 366 us, 500 543 -> 412, 750 557 -> 452, 1000 550 -> 504,
+// 1250 599 -> 592, 2000 unchanged; forward T = 500 166 -> 137; without a shared
+// expert T = 2000 463 -> 433.  Fewer tiles (130, 160) lose most of it (T = 500
+// 503, T = 1000 552), more (260) cost T = 2000 662 -> 716, no limit costs T =
+// 1500, E = 64, k = 6 forward 369 -> 389.  More full rows (130) cost T = 2646, H =
+// 840, E = 8, I = S = 1936 559 -> 568 (its dense tiles are full), fewer (90) lose
+// T = 1000.
+constexpr double kBusyTiles = 200, kBusyRows = 110;
+struct TileCost {
+  double one, two;
+};
+struct TileCosts {
+  double big;  // a round of 256-row tiles
+  TileCost mid, small;
+};
+constexpr TileCosts kGateUpCosts{10.0, {5.2, 7.0}, {3.1, 4.7}};
+constexpr TileCosts kGemmCosts{10.0, {6.8, 8.2}, {4.4, 5.7}};
+constexpr TileCosts kSwigluBwdCosts{12.0, {6.8, 8.2}, {5.0, 6.2}};  // down input gradient
+// A 384-row tile against a 256-row one (a k-tile brings 25 % more operand rows
+// for 50 % more MFMA work).
+constexpr double kRows384Cost = 1.4;
+
+double round_cost(double tiles, const TileCost& c) {
+  const double full = std::floor(tiles / 512.0), rest = tiles - 512.0 * full;
+  return full * c.two + (rest <= 0.0 ? 0.0 : rest <= 256.0 ? c.one : c.two);
+}
+double big_cost(double tiles, double c) { return std::ceil(tiles / 256.0) * c; }
+// Row tiles of height bm over E groups of r rows on average.
+double group_row_tiles(int E, double r, int bm) { return E * std::max(1.0, r / bm + 0.5); }
+// Whether a routed launch over n_routed columns (in tiles of bn) and the shared
+// expert's over n_shared columns beside it leave CUs idle on 256-row tiles:
+// fewer than kBusyTiles of them, holding fewer rows than kBusyRows full ones.
+bool leaves_idle(const moe_config& c, int64_t T, int n_routed, int n_shared, int bn) {
+  const int64_t TK = T * c.experts_per_tok;
+  const int groups = (int)std::min<int64_t>(c.num_experts, TK);
+  const double sh = c.shared_intermediate > 0 ? ceil_div(n_shared, bn) : 0;
+  const double tiles = group_row_tiles(groups, (double)TK / groups, 256) * ceil_div(n_routed, bn) +
+                       ceil_div(T, 256) * sh;
+  const double full = (TK * (double)ceil_div(n_routed, bn) + T * sh) / 256.0;
+  return tiles < kBusyTiles && full < kBusyRows;
 }
 
+// Calls f(tiling, grid) for a dense (shared-expert) launch of tiling C over T
+// rows and N columns: C, its 384-row tiles or one of the shorter tilings,
+// whichever costs least.  The last row tile of C or its 384-row tiles runs as
+// the shortest tiling that covers it.  idle: leaves_idle of it and the routed
+// launch beside it.  MID = false (the launches over H columns): such a launch
+// that leaves CUs idle holds at most 440 64 x 128 tiles, fewer than a round.
+template <typename D, class C, bool MID, class F>
+void with_dense_tiling(int T, int N, const TileCosts& cost, bool idle, F&& f) {
+  auto tiles = [&](auto c) {
+    using CC = decltype(c);
+    return (int64_t)ceil_div(T, CC::AR) * ceil_div(N, CC::BN);
+  };
+  auto go = [&](auto c) { f(c, (int)tiles(c)); };
+  if constexpr (has_half_rows<D, C>()) {
+    using C3 = Rows384<C>;
+    using CM = typename LowTilings<C>::Mid;
+    using CS = typename LowTilings<C>::Small;
+    const double big = big_cost((double)tiles(C{}), cost.big);
+    const double tall = big_cost((double)tiles(C3{}), cost.big * kRows384Cost);
+    const double small = round_cost((double)tiles(CS{}), cost.small);
+    const double mid = MID ? round_cost((double)tiles(CM{}), cost.mid) : small;
+    double best = std::min(big, tall);
+    if (idle) best = std::min(best, std::min(mid, small));
+    if (best < big) {
+      if (tall == best) return go(C3{});
+      if constexpr (MID) {
+        if (mid == best) return go(CM{});
+      }
+      return go(CS{});
+    }
+  }
+  go(C{});
+}
+
+// Shared expert forward over all T tokens on stream ss: G, U (when kept), A,
+// and the down projection into sY when sY is not null.
 template <typename D>
 void shared_fwd(moe_plan* p, hipStream_t ss, int T, const D* x, const moe_weights* w, D* sG,
                 D* sU, D* sA, D* sY) {
@@ -793,14 +875,15 @@ void shared_fwd(moe_plan* p, hipStream_t ss, int T, const D* x, const moe_weight
     else go(std::integral_constant<int, 4>());
   } else {
     const RowGroups dense{nullptr, nullptr, nullptr, nullptr, 1, T, 0, 0};
-    with_dense_tiling<D, CG>(T, S, [&](auto c, int grid) {
+    const moe_config& c = p->cfg;
+    with_dense_tiling<D, CG, true>(T, S, kGateUpCosts, leaves_idle(c, T, c.intermediate, S, CG::BN), [&](auto c, int grid) {
       using C = decltype(c);
       hipLaunchKernelGGL((k_gateup_fwd<D, false, C>), dim3(grid), dim3(C::THREADS), 0, ss, x, dense,
                          nullptr, (const D*)w->shared_gate, nullptr, (const D*)w->shared_up, H, S,
                          sG, sU, sA, nullptr, 0, 1);
     });
     if (sY)
-      with_dense_tiling<D, CB>(T, H, [&](auto c, int grid) {
+      with_dense_tiling<D, CB, false>(T, H, kGemmCosts, leaves_idle(c, T, H, H, CB::BN), [&](auto c, int grid) {
         using C = decltype(c);
         hipLaunchKernelGGL((k_down_fwd<D, false, C>), dim3(grid), dim3(C::THREADS), 0, ss, sA, dense,
                            nullptr, (const D*)w->shared_down, S, H, sY, nullptr);
@@ -813,18 +896,27 @@ void shared_fwd(moe_plan* p, hipStream_t ss, int T, const D* x, const moe_weight
 // tiles save.
 constexpr int kRows384Rounds = 4;
 
-// Calls f(tiling, row groups, grid(N)) for a row-grouped launch of tiling C
-// with N output columns: the tile prefixes of C::BM, and a grid
-// of the row-tile upper bound TK / BM + E times the column tiles, rounded up
-// to whole rounds of the 8 XCDs (xcd_slot2).  Half tiles run last when they
+// Calls f(tiling, row groups, grid) for a row-grouped launch of tiling C (or
+// the taller or shorter one picked for it) with N output columns: the tile
+// prefixes of its height, and a grid of the row-tile upper bound TK / BM + E
+// times the column tiles, rounded up to whole rounds of the 8 XCDs
+// (xcd_slot2).  Half tiles run last when they
 // have a half-height tiling and the groups average at least two row tiles:
 // with fewer rows per expert (config 5: 256) the weight panels dominate the
 // traffic, and a half tile that runs apart from its expert's big tiles reads
 // them again (measured: config 2 gate/up forward 296 -> 249 us, config 5
 // row-grouped GEMMs 3-4 % slower).
 template <typename D, class C, bool ROWS384 = true, class F>
-void with_row_tiling(const int* offsets, const int* tprefix_all, int E, int64_t TK, F&& f) {
-  if constexpr (ROWS384 && has_half_rows<D, C>()) {
+void with_row_tiling(const int* offsets, const int* tprefix_all, int E, int64_t TK, int N,
+                     const TileCosts& cost, bool idle, F&& f) {
+  auto go = [&](auto c, int half_last, int tall) {
+    using CC = decltype(c);
+    const int* tp = tprefix_all + prefix_slot(CC::XR == 128 ? CC::AR : CC::BM) * (E + 1);
+    const int mt = ceil_div(TK, CC::XR == 128 ? CC::AR : CC::BM) + E;
+    f(c, RowGroups{offsets, tp, tp + (E + 1), tp + 2 * (E + 1), E, (int)TK, half_last, tall},
+      8 * ceil_div((int64_t)mt * ceil_div(N, CC::BN), 8));
+  };
+  if constexpr (has_half_rows<D, C>()) {
     // 384-row tiles, the half tiles (at most 192 rows) after the big ones,
     // when the groups average at least two of them and the launch holds at
     // least four rounds of them over 256 CUs at six column tiles (I = 1408):
@@ -834,24 +926,25 @@ void with_row_tiling(const int* offsets, const int* tprefix_all, int E, int64_t 
     // input gradient keeps 256-row tiles (ROWS384 = false: config 3 0.86 ->
     // 0.89 ms with them).
     using C3 = Rows384<C>;
-    if (TK >= 2 * (int64_t)C3::AR * E && 6 * TK >= (int64_t)kRows384Rounds * 256 * C3::AR) {
-      const int* tp = tprefix_all + kTilePrefixes * tile_slot(C3::AR) * (E + 1);
-      const int mt = ceil_div(TK, C3::AR) + E;
-      static_assert(tall_rows_for(C3::AR) == 0, "384-row tiles take no tails");
-      f(C3{}, RowGroups{offsets, tp, tp + (E + 1), tp + 2 * (E + 1), E, (int)TK, 1, 0},
-        [mt](int N) { return 8 * ceil_div(mt * ceil_div(N, C3::BN), 8); });
-      return;
-    }
+    static_assert(C3::AR == 384 && tall_rows_for(C3::AR) == 0, "384-row tiles take no tails");
+    if (ROWS384 && TK >= 2 * (int64_t)C3::AR * E && 6 * TK >= (int64_t)kRows384Rounds * 256 * C3::AR)
+      return go(C3{}, 1, 0);
+    using CM = typename LowTilings<C>::Mid;
+    using CS = typename LowTilings<C>::Small;
+    const int groups = (int)std::min<int64_t>(E, TK);
+    const double r = (double)TK / groups;
+    const double big =
+        big_cost(group_row_tiles(groups, r, C::BM) * ceil_div(N, C::BN), cost.big) / 1.15;
+    const double mid =
+        round_cost(group_row_tiles(groups, r, CM::BM) * ceil_div(N, CM::BN), cost.mid);
+    const double small =
+        round_cost(group_row_tiles(groups, r, CS::BM) * ceil_div(N, CS::BN), cost.small);
+    if (idle && std::min(mid, small) < big) return mid <= small ? go(CM{}, 0, 0) : go(CS{}, 0, 0);
   }
-  const int* tp = tprefix_all + kTilePrefixes * tile_slot(C::BM) * (E + 1);
-  const int mt = ceil_div(TK, C::BM) + E;
-  const int half_last = has_half_rows<D, C>() && TK >= 2 * (int64_t)C::BM * E;
   // the prefixes (k_scan) merge short tails into tall tiles exactly where the
   // kernels' row tilings have them
   static_assert(tall_rows_for(C::BM) == (has_half_rows<D, C>() ? C::BM / 4 : 0), "tall tiles");
-  f(C{}, RowGroups{offsets, tp, tp + (E + 1), tp + 2 * (E + 1), E, (int)TK, half_last,
-                   tall_rows_for(C::BM)},
-    [mt](int N) { return 8 * ceil_div(mt * ceil_div(N, C::BN), 8); });
+  go(C{}, has_half_rows<D, C>() && TK >= 2 * (int64_t)C::BM * E, tall_rows_for(C::BM));
 }
 
 // Routed experts forward on stream s: G, U (when kept), A and the
@@ -895,9 +988,9 @@ moe_status routed_fwd(moe_plan* p, hipStream_t s, int T, const D* x, const State
       if (T <= 16) go(std::integral_constant<int, 1>());
       else go(std::integral_constant<int, 4>());
     } else {
-      with_row_tiling<D, CG>(st.offsets, st.tprefix, E, TK, [&](auto c, const RowGroups& r, auto grid) {
+      with_row_tiling<D, CG>(st.offsets, st.tprefix, E, TK, I, kGateUpCosts, leaves_idle(c, T, I, c.shared_intermediate, CG::BN), [&](auto c, const RowGroups& r, int grid) {
         using C = decltype(c);
-        hipLaunchKernelGGL((k_gateup_fwd<D, true, C>), dim3(grid(I)), dim3(C::THREADS), 0,
+        hipLaunchKernelGGL((k_gateup_fwd<D, true, C>), dim3(grid), dim3(C::THREADS), 0,
                            s, x, r, tg, nullptr, tu, nullptr, H, I, st.G, st.U, st.A, st.perm,
                            T, k);
       });
@@ -918,9 +1011,9 @@ moe_status routed_fwd(moe_plan* p, hipStream_t s, int T, const D* x, const State
       if (T <= 16) go(std::integral_constant<int, 1>());
       else go(std::integral_constant<int, 4>());
     } else {
-      with_row_tiling<D, CB>(st.offsets, st.tprefix, E, TK, [&](auto c, const RowGroups& r, auto grid) {
+      with_row_tiling<D, CB>(st.offsets, st.tprefix, E, TK, H, kGemmCosts, leaves_idle(c, T, H, H, CB::BN), [&](auto c, const RowGroups& r, int grid) {
         using C = decltype(c);
-        hipLaunchKernelGGL((k_down_fwd<D, true, C>), dim3(grid(H)), dim3(C::THREADS), 0, s,
+        hipLaunchKernelGGL((k_down_fwd<D, true, C>), dim3(grid), dim3(C::THREADS), 0, s,
                            st.A, r, td, nullptr, I, H, st.Y, st.perm);
       });
     }
@@ -1166,13 +1259,13 @@ moe_status backward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* dout,
     dxs = (D*)(ws + W.dxs);
     const float sc = c.shared_expert_scale;
     const RowGroups dense{nullptr, nullptr, nullptr, nullptr, 1, T, 0, 0};
-    with_dense_tiling<D, CB>(T, S, [&](auto c, int grid) {
+    with_dense_tiling<D, CB, true>(T, S, kSwigluBwdCosts, leaves_idle(c, T, I, S, CB::BN), [&](auto c, int grid) {
       using C = decltype(c);
       hipLaunchKernelGGL((k_down_dgrad<D, false, C>), dim3(grid), dim3(C::THREADS), 0, ss, dout,
                          dense, nullptr, (const D*)w->shared_down, H, S, sc, sG, sU, sdG, sdU,
                          nullptr, 0, 1, nullptr);
     });
-    with_dense_tiling<D, CB>(T, H, [&](auto c, int grid) {
+    with_dense_tiling<D, CB, false>(T, H, kGemmCosts, leaves_idle(c, T, H, H, CB::BN), [&](auto c, int grid) {
       using C = decltype(c);
       hipLaunchKernelGGL((k_gateup_dgrad<D, false, C>), dim3(grid), dim3(C::THREADS), 0, ss, sdG,
                          sdU, dense, nullptr, (const D*)w->shared_gate, nullptr,
@@ -1245,9 +1338,9 @@ moe_status backward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* dout,
   }
   {
     StageTimer tm(p, s, MOE_STAGE_DOWN_DGRAD);
-    with_row_tiling<D, CB, false>(offsets, st.tprefix, E, TK, [&](auto c, const RowGroups& r, auto grid) {
+    with_row_tiling<D, CB, false>(offsets, st.tprefix, E, TK, I, kSwigluBwdCosts, leaves_idle(c, T, I, S, CB::BN), [&](auto c, const RowGroups& r, int grid) {
       using C = decltype(c);
-      hipLaunchKernelGGL((k_down_dgrad<D, true, C>), dim3(grid(I)), dim3(C::THREADS), 0, s,
+      hipLaunchKernelGGL((k_down_dgrad<D, true, C>), dim3(grid), dim3(C::THREADS), 0, s,
                          dout, r, td, nullptr, H, I, 1.0f, G, U, dG, dU, st.perm, T, k, dwp);
     });
     LAUNCH_CHECK();
@@ -1284,9 +1377,9 @@ moe_status backward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* dout,
   }
   {
     StageTimer tm(p, s, MOE_STAGE_GATEUP_DGRAD);
-    with_row_tiling<D, CB>(offsets, st.tprefix, E, TK, [&](auto c, const RowGroups& r, auto grid) {
+    with_row_tiling<D, CB>(offsets, st.tprefix, E, TK, H, kGemmCosts, leaves_idle(c, T, H, H, CB::BN), [&](auto c, const RowGroups& r, int grid) {
       using C = decltype(c);
-      hipLaunchKernelGGL((k_gateup_dgrad<D, true, C>), dim3(grid(H)), dim3(C::THREADS), 0,
+      hipLaunchKernelGGL((k_gateup_dgrad<D, true, C>), dim3(grid), dim3(C::THREADS), 0,
                          s, dG, dU, r, tg, nullptr, tu, nullptr, I, H, dXp, st.perm);
     });
     LAUNCH_CHECK();
