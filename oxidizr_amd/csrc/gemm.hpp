@@ -2,11 +2,9 @@
 //
 // One workgroup of 4 or 8 wave64s (Tiling::NW) in a WGM x WGN arrangement
 // computes a BM x BN output tile of  C[m, n] = sum_k A(m, k) * B(n, k).
-// Operands are staged through LDS as K-contiguous rows ([row][k], padded by
-// one 16-byte vector per row against bank conflicts). An operand whose memory
-// layout is K-major ("transposed": element (r, k) at base + k * ld + r) is
-// turned into that LDS layout with an in-register V x V transpose, so the
-// MFMA fragment reads are always one ds_read_b128 per lane.
+// Operands are streamed into LDS by direct-to-LDS loads, as K-contiguous rows
+// ([row][k]) or, for an operand whose memory layout is K-major ("transposed":
+// element (r, k) at base + k * ld + r), as k-rows.
 //
 // The MFMA "row" input is fed from the B tile and the "column" input from the
 // A tile, so the accumulator D[i][j] holds C[m = j][n = i]: each lane then
@@ -40,7 +38,6 @@ struct Tiling {
   static constexpr int BM = BM_, BN = BN_, BK = BK_;
   static constexpr int NST = NST_;        // LDS pipeline stages (direct-to-LDS loop)
   static constexpr int V = Vec16<T>::N;   // elements per 16-byte vector
-  static constexpr int LDK = BK + V;      // padded LDS row pitch (elements)
   static constexpr int NW = NW_;          // waves per workgroup
   static constexpr int THREADS = 64 * NW;
   static constexpr int WGN = WGN_, WGM = NW_ / WGN_;  // wave grid
@@ -109,134 +106,6 @@ MOE_DEV void mfma_frag(f32x16& acc, u32x4 bt, u32x4 at, float) {
   acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(bt.w), __uint_as_float(at.w), acc, 0, 0, 0);
 }
 
-// V x V transpose of 16-byte row vectors: out[c] element i = in[i] element c.
-MOE_DEV void transpose_vv(const u32x4 (&in)[8], u32x4 (&out)[8], bf16_t) {
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {      // source word q holds elements 2q (low) and 2q+1 (high)
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {    // destination word w holds rows 2w (low) and 2w+1 (high)
-      uint32_t a = in[2 * w][q], b = in[2 * w + 1][q];
-      out[2 * q][w] = (a & 0xffffu) | (b << 16);
-      out[2 * q + 1][w] = (a >> 16) | (b & 0xffff0000u);
-    }
-  }
-}
-MOE_DEV void transpose_vv(const u32x4 (&in)[4], u32x4 (&out)[4], float) {
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) out[c][i] = in[i][c];
-}
-
-// Per-thread staging of one operand tile of R rows between global memory and
-// LDS.  Loads are raw buffer loads: the resource covers exactly the operand's
-// readable extent, so out-of-range rows and the K tail come back as zero from
-// the hardware (no per-load branches), the tile base sits in scalar registers
-// and each load needs one 32-bit offset register.
-template <class C, typename T, int R, bool TRANS, bool G = false>
-struct Stager;
-
-template <class C, typename T, int R, bool G>
-struct Stager<C, T, R, false, G> {
-  static constexpr int KV = C::BK / C::V;              // vectors per row
-  static constexpr int TOTAL = R * KV;
-  static_assert(TOTAL % C::THREADS == 0, "tile rows must cover the workgroup");
-  static constexpr int PER = TOTAL / C::THREADS;
-  static constexpr int ROWS_STEP = C::THREADS / KV;    // rows between a thread's loads
-  u32x4 r[PER];
-  rsrc_t rs[2];                                        // one per K segment
-  int k_valid[2];
-  uint32_t voff, step;
-  uint32_t vrow[G ? PER : 1];                          // gathered: each load's row offset
-  int kcol;
-  MOE_DEV static rsrc_t rsrc_of(const OpDesc<T>& d) {
-    const int64_t limit = G ? (int64_t)d.src_rows * d.ld
-                            : (int64_t)(d.rows_valid - 1) * d.ld + d.k_valid;
-    return make_rsrc(d.base, (uint32_t)(limit * (int64_t)sizeof(T)));
-  }
-  MOE_DEV void init(const OpDesc<T>& d, int tid) {
-    rs[0] = rs[1] = rsrc_of(d);
-    k_valid[0] = k_valid[1] = d.k_valid;
-    kcol = (tid % KV) * C::V;
-    voff = (uint32_t)(((tid / KV) * d.ld + kcol) * (int64_t)sizeof(T));
-    step = (uint32_t)(ROWS_STEP * d.ld * (int64_t)sizeof(T));
-    if constexpr (G) {
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        vrow[i] = gathered_row_offset(d, tid / KV + i * ROWS_STEP, kcol);
-      }
-    }
-  }
-  // Second K segment: same ld and rows as the first.
-  MOE_DEV void init_second(const OpDesc<T>& d) {
-    rs[1] = rsrc_of(d);
-    k_valid[1] = d.k_valid;
-  }
-  MOE_DEV void load(int k0, int seg) {
-    const uint32_t soff = (uint32_t)k0 * sizeof(T);
-    const bool kin = k0 + kcol < k_valid[seg];
-#pragma unroll
-    for (int i = 0; i < PER; ++i)
-      r[i] = buf_ld16(rs[seg], kin ? (G ? vrow[i] : voff + i * step) : kOobOffset, soff);
-  }
-  MOE_DEV void store(T* s, int tid) const {
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int c = tid + i * C::THREADS;
-      const int row = c / KV, kv = c % KV;
-      st16(s + row * C::LDK + kv * C::V, r[i]);
-    }
-  }
-};
-
-template <class C, typename T, int R>
-struct Stager<C, T, R, true> {
-  static constexpr int V = C::V;
-  static constexpr int RB = R / V, KB = C::BK / V;     // V x V blocks
-  static constexpr int TOTAL = RB * KB;
-  static constexpr int PER = (TOTAL + C::THREADS - 1) / C::THREADS;
-  u32x4 r[PER][V];
-  rsrc_t rs[2];                                        // one per K segment
-  uint32_t voff, ldb;
-  MOE_DEV static rsrc_t rsrc_of(const OpDesc<T>& d) {
-    const int rv = (d.rows_valid + V - 1) / V * V;
-    const int64_t limit = (int64_t)(d.k_valid - 1) * d.ld + rv;
-    return make_rsrc(d.base, d.k_valid > 0 ? (uint32_t)(limit * (int64_t)sizeof(T)) : 0u);
-  }
-  MOE_DEV void init(const OpDesc<T>& d, int tid) {
-    rs[0] = rs[1] = rsrc_of(d);
-    const int rb = tid % RB, kb = tid / RB;            // adjacent threads: adjacent rows
-    voff = (uint32_t)(((int64_t)kb * V * d.ld + rb * V) * (int64_t)sizeof(T));
-    ldb = (uint32_t)(d.ld * (int64_t)sizeof(T));
-  }
-  // Second K segment: same ld and rows as the first.
-  MOE_DEV void init_second(const OpDesc<T>& d) { rs[1] = rsrc_of(d); }
-  MOE_DEV void load(int k0, int seg) {
-    const uint32_t soff = (uint32_t)k0 * ldb;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      if (TOTAL % C::THREADS == 0 || (int)threadIdx.x + i * C::THREADS < TOTAL) {
-        const uint32_t vi = voff + (uint32_t)(i * (C::THREADS / RB) * V) * ldb;
-#pragma unroll
-        for (int j = 0; j < V; ++j) r[i][j] = buf_ld16(rs[seg], vi + j * ldb, soff);
-      }
-    }
-  }
-  MOE_DEV void store(T* s, int tid) const {
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int b = tid + i * C::THREADS;
-      if (TOTAL % C::THREADS == 0 || b < TOTAL) {
-        const int rb = b % RB, kb = b / RB;
-        u32x4 t[V];
-        transpose_vv(r[i], t, T());
-#pragma unroll
-        for (int c = 0; c < V; ++c) st16(s + (rb * V + c) * C::LDK + kb * C::V, t[c]);
-      }
-    }
-  }
-};
-
 // ---------------------------------------------------------------------------
 // Direct-to-LDS path.  Buffer loads with the LDS modifier stream 16-byte
 // vectors from global memory straight into LDS (no staging registers, no
@@ -250,9 +119,10 @@ struct Stager<C, T, R, true> {
 // different ones as well).  The lane that fills slot s of row r therefore
 // loads k-vector s ^ nt_swz(r).
 //
-// K-major operand tile (bf16 only; element (r, k) at base + k*ld + r): BK
-// k-rows of R contiguous columns; the 16-byte slot p of k-row k sits at
-// p ^ tr_swz(k).  Fragments come from ds_read_b64_tr_b16: within each group of
+// K-major operand tile (element (r, k) at base + k*ld + r): BK k-rows of R
+// contiguous columns.  fp32: unswizzled rows, fragments by four ds_read_b32
+// down a column (DmaStagerT32).  bf16: the 16-byte slot p of k-row k sits at
+// p ^ tr_swz(k) and fragments come from ds_read_b64_tr_b16: within each group of
 // 16 lanes, lane 4i + j receives in slot q element j of the 8-byte chunk
 // addressed by lane 4q + i.  When lane 4q + i of group b addresses k-row
 // kk + 8 (b >> 1) + q at column c0 + 16 (b & 1) + 4i, lane L receives the four
@@ -373,6 +243,55 @@ struct DmaStagerT {
   }
 };
 
+// fp32 K-major operand: a lane needs one float per MFMA, so a fragment is a
+// column of the k-rows as they lie in memory, 32 consecutive floats to a
+// half-wave, and nothing is transposed.  Before, these operands were staged
+// through registers with a 4 x 4 transpose into padded rows.  Launches alone, 12
+// experts of 500 rows (H = 776, I = 1368): gate/up input gradient 305 -> 262 us,
+// weight gradients 152 -> 118 and 305 -> 261; config 1 (8 of 256 rows, H = 384, I
+// = 1024): 54 -> 46, 24 -> 19 and 49 -> 42 us; same bits.
+template <class C, int R>
+struct DmaStagerT32 {
+  static constexpr int SPR = R / 4;              // 16-byte slots per k-row
+  static_assert(SPR >= 8 && SPR <= 64 && 64 % SPR == 0, "K-major tiles of 32 to 256 columns");
+  static constexpr int RPI = 64 / SPR;           // k-rows per 1 KB instruction
+  static constexpr int PER = C::BK / (C::NW * RPI);  // instructions per wave per k-tile
+  static_assert(PER >= 1 && C::BK % (C::NW * RPI) == 0, "k-rows must cover the waves");
+  rsrc_t rs[2];
+  uint32_t voff, ldb;
+  MOE_DEV static rsrc_t rsrc_of(const OpDesc<float>& d) {
+    const int rv = (d.rows_valid + 3) / 4 * 4;
+    const int64_t limit = (int64_t)(d.k_valid - 1) * d.ld + rv;
+    return make_rsrc(d.base, d.k_valid > 0 ? (uint32_t)(limit * 4) : 0u);
+  }
+  MOE_DEV void init(const OpDesc<float>& d, int tid) {
+    rs[0] = rs[1] = rsrc_of(d);
+    const int lane = tid & 63, wave = tid >> 6;
+    voff = (uint32_t)(((int64_t)(wave * RPI + lane / SPR) * d.ld + (lane % SPR) * 4) * 4);
+    ldb = (uint32_t)(d.ld * 4);
+  }
+  MOE_DEV void init_second(const OpDesc<float>& d) { rs[1] = rsrc_of(d); }
+  MOE_DEV void issue(float* tile, int k0, int seg) const {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rs[seg], (lds_void_t*)(tile + (i * C::NW * RPI + wave * RPI) * R), 16,
+          voff + (uint32_t)(i * C::NW * RPI) * ldb, (uint32_t)k0 * ldb, 0, 0);
+  }
+  // component c: k = kk + 4 (lane / 32) + c of column col0 + lane % 32, the k
+  // slots of a K-contiguous operand's 16-byte fragment
+  MOE_DEV static u32x4 frag(const float* tile, int col0, int kk) {
+    const int lane = threadIdx.x & 63;
+    const float* a = tile + (kk + 4 * (lane >> 5)) * R + col0 + (lane & 31);
+    return u32x4{__float_as_uint(a[0]), __float_as_uint(a[R]), __float_as_uint(a[2 * R]),
+                 __float_as_uint(a[3 * R])};
+  }
+};
+template <class C, typename T, int R>
+using KMajorStager = typename std::conditional<sizeof(T) == 4, DmaStagerT32<C, R>,
+                                               DmaStagerT<C, bf16_t, R>>::type;
+
 // acc += B x A over K with both operands fed by DMA into C::NST unpadded LDS
 // stages (k-tile kt in stage kt % NST).  While k-tile kt is multiplied out,
 // the DMA of the next NST - 1 k-tiles is in flight.  Before k-tile kt + 1 is
@@ -420,8 +339,8 @@ MOE_DEV void mainloop_dma(f32x16 (&acc)[NA * NB][C::TN][C::TM],
   constexpr bool TALL = C::XR > 0;
   static_assert(!TALL || !A_T, "tall tiles take a K-contiguous A operand");
   static_assert(!AG || !A_T, "gathered rows: K-contiguous A");
-  using SA = typename std::conditional<A_T, DmaStagerT<C, T, C::AR>, DmaStager<C, T, C::AR, AG>>::type;
-  using SB = typename std::conditional<B_T, DmaStagerT<C, T, C::BN>, DmaStager<C, T, C::BN>>::type;
+  using SA = typename std::conditional<A_T, KMajorStager<C, T, C::AR>, DmaStager<C, T, C::AR, AG>>::type;
+  using SB = typename std::conditional<B_T, KMajorStager<C, T, C::BN>, DmaStager<C, T, C::BN>>::type;
   // DMA instructions one wave issues per k-tile
   constexpr int IPT = NA * SA::PER + NB * SB::PER;
   static_assert((NST - 2) * IPT <= 63, "vmcnt range");
@@ -470,7 +389,7 @@ MOE_DEV void mainloop_dma(f32x16 (&acc)[NA * NB][C::TN][C::TM],
     for (int i = 0; i < NA; ++i) {
 #pragma unroll
       for (int tm = 0; tm < C::TM; ++tm) {
-        if constexpr (A_T) af[set][i][tm] = SA::frag(sA + i * TILE_A, wm * C::WM + tm * 32, ks * 16);
+        if constexpr (A_T) af[set][i][tm] = SA::frag(sA + i * TILE_A, wm * C::WM + tm * 32, ks * 2 * C::V);
         else af[set][i][tm] = SA::frag(sA + i * TILE_A, wm * C::WM + tm * 32 + frag_row, kv);
       }
       if constexpr (TALL) afx[set][i] = SA::frag(sA + i * TILE_A, xrow, kv);
@@ -479,7 +398,7 @@ MOE_DEV void mainloop_dma(f32x16 (&acc)[NA * NB][C::TN][C::TM],
     for (int i = 0; i < NB; ++i)
 #pragma unroll
       for (int tn = 0; tn < C::TN; ++tn) {
-        if constexpr (B_T) bfr[set][i][tn] = SB::frag(sB + i * TILE_B, wn * C::WN + tn * 32, ks * 16);
+        if constexpr (B_T) bfr[set][i][tn] = SB::frag(sB + i * TILE_B, wn * C::WN + tn * 32, ks * 2 * C::V);
         else bfr[set][i][tn] = SB::frag(sB + i * TILE_B, wn * C::WN + tn * 32 + frag_row, kv);
       }
   };
@@ -605,131 +524,20 @@ MOE_DEV void mainloop_dma(f32x16 (&acc)[NA * NB][C::TN][C::TM],
   __syncthreads();  // the caller's epilogue reuses the LDS
 }
 
-// LDS elements of one pipeline stage and of the whole (double-buffered)
-// main loop with NA A operands and NB B operands.
+// LDS elements of the main loop's stages with NA A operands and NB B operands.
 template <class C, int NA, int NB>
-constexpr int stage_elems() { return (NA * C::BM + NB * C::BN) * C::LDK; }
-// 16-bit operands always take the direct-to-LDS loop, whose tiles are
-// unpadded; fp32 keeps the padded pitch of the register-staged loop.
-template <class C, int NA, int NB>
-constexpr int smem_elems() {
-  return C::V == 8 ? C::NST * (NA * C::AR + NB * C::BN) * C::BK : 2 * stage_elems<C, NA, NB>();
-}
+constexpr int smem_elems() { return C::NST * (NA * C::AR + NB * C::BN) * C::BK; }
 
-// acc[a * NB + b][tn][tm] += B_b-tile x A_a-tile over k in [0, K).
-// Two LDS stages: while the waves multiply out of stage kt & 1, the k-tile
-// kt + 1 (fetched into registers one iteration earlier) is written to the
-// other stage and k-tile kt + 2 is fetched from global memory, so each global
-// load has a whole iteration of MFMA work to land and every iteration needs a
-// single barrier.
-//
-// An optional second K segment (a2, b2, K2: same ld and rows as a and b)
-// continues the same pipeline, so sum_k A1 B1 + sum_k A2 B2 runs as one loop.
+// acc[a * NB + b][tn][tm] += B_b-tile x A_a-tile over k in [0, K).  An optional
+// second K segment (a2, b2, K2: same ld and rows as a and b) continues the same
+// pipeline, so sum_k A1 B1 + sum_k A2 B2 runs as one loop.
 template <class C, typename T, bool A_T, bool B_T, int NA, int NB, bool AG = false>
 MOE_DEV void mainloop(f32x16 (&acc)[NA * NB][C::TN][C::TM], const OpDesc<T> (&a)[NA],
                       const OpDesc<T> (&b)[NB], int K, T* smem, const OpDesc<T>* a2 = nullptr,
                       const OpDesc<T>* b2 = nullptr, int K2 = 0) {
-  // DMA for every bf16 operand layout; fp32 K-major operands keep the
-  // register-staged transpose below (the transposing LDS read is 16-bit)
   static_assert(C::XR == 0, "tall tiles run mainloop_x");
-  if constexpr (sizeof(T) == 2 || (!A_T && !B_T)) {
-    static_assert(C::NST * (NA * C::BM + NB * C::BN) * C::BK <= smem_elems<C, NA, NB>(), "LDS");
-    f32x16 unused[NA * NB][C::XTN];
-    mainloop_dma<C, T, A_T, B_T, NA, NB, AG>(acc, unused, a, b, K, smem, a2, b2, K2);
-    return;
-  }
-  constexpr int STAGE = stage_elems<C, NA, NB>();
-  constexpr int B_OFF = NA * C::BM * C::LDK;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / C::WGN, wn = wave % C::WGN;
-  static_assert(!AG || !A_T, "gathered rows: K-contiguous A");
-  Stager<C, T, C::BM, A_T, AG> sa[NA];
-  Stager<C, T, C::BN, B_T> sb[NB];
-  const int nk1 = (K + C::BK - 1) / C::BK;
-  const int nk = nk1 + (K2 > 0 ? (K2 + C::BK - 1) / C::BK : 0);
-  if (nk <= 0) return;
-
-#pragma unroll
-  for (int i = 0; i < NA; ++i) {
-    sa[i].init(a[i], tid);
-    if (K2 > 0) sa[i].init_second(a2[i]);
-  }
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    sb[i].init(b[i], tid);
-    if (K2 > 0) sb[i].init_second(b2[i]);
-  }
-  auto fetch = [&](int kt) {
-    const int seg = kt >= nk1 ? 1 : 0;
-    const int k0 = (kt - seg * nk1) * C::BK;
-#pragma unroll
-    for (int i = 0; i < NA; ++i) sa[i].load(k0, seg);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) sb[i].load(k0, seg);
-  };
-  auto put = [&](T* stage) {
-#pragma unroll
-    for (int i = 0; i < NA; ++i) sa[i].store(stage + i * C::BM * C::LDK, tid);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) sb[i].store(stage + B_OFF + i * C::BN * C::LDK, tid);
-  };
-
-  fetch(0);
-  put(smem);
-  if (nk > 1) fetch(1);
-  __syncthreads();
-
-  const int frag_row = lane & 31;
-  const int frag_k = (lane >> 5) * C::V;
-  constexpr int KSTEPS = C::BK / (2 * C::V);
-  // Fragments of one k-step; two register sets so the LDS reads of step
-  // kk + 1 are in flight while the MFMAs of step kk issue.
-  u32x4 af[2][NA][C::TM], bfr[2][NB][C::TN];
-  auto read_frags = [&](const T* sA, const T* sB, int kk, int set) {
-#pragma unroll
-    for (int i = 0; i < NA; ++i)
-#pragma unroll
-      for (int tm = 0; tm < C::TM; ++tm)
-        af[set][i][tm] = *reinterpret_cast<const u32x4*>(
-            sA + i * C::BM * C::LDK + (wm * C::WM + tm * 32 + frag_row) * C::LDK + kk + frag_k);
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-#pragma unroll
-      for (int tn = 0; tn < C::TN; ++tn)
-        bfr[set][i][tn] = *reinterpret_cast<const u32x4*>(
-            sB + i * C::BN * C::LDK + (wn * C::WN + tn * 32 + frag_row) * C::LDK + kk + frag_k);
-  };
-  for (int kt = 0; kt < nk; ++kt) {
-    const T* sA = smem + (kt & 1) * STAGE;
-    const T* sB = sA + B_OFF;
-    read_frags(sA, sB, 0, 0);
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-      const int cur = ks & 1;
-      if (ks + 1 < KSTEPS) read_frags(sA, sB, (ks + 1) * 2 * C::V, cur ^ 1);
-#pragma unroll
-      for (int ia = 0; ia < NA; ++ia)
-#pragma unroll
-        for (int ib = 0; ib < NB; ++ib)
-#pragma unroll
-          for (int tn = 0; tn < C::TN; ++tn)
-#pragma unroll
-            for (int tm = 0; tm < C::TM; ++tm)
-              mfma_frag(acc[ia * NB + ib][tn][tm], bfr[cur][ib][tn], af[cur][ia][tm], T());
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (kt + 1 < nk) {
-      // stage (kt + 1) & 1 was last read in iteration kt - 1, which every
-      // wave finished before the barrier that closed that iteration
-      put(smem + ((kt + 1) & 1) * STAGE);
-      // keep the next fetch below the stores: hoisting it would need a
-      // second set of staging registers
-      __builtin_amdgcn_sched_barrier(0);
-      if (kt + 2 < nk) fetch(kt + 2);
-    }
-    __syncthreads();
-  }
+  f32x16 unused[NA * NB][C::XTN];
+  mainloop_dma<C, T, A_T, B_T, NA, NB, AG>(acc, unused, a, b, K, smem, a2, b2, K2);
 }
 
 // mainloop for a row tile that may be tall (C::XR > 0, bf16): xacc holds the

@@ -63,23 +63,28 @@ struct LowTilings {
   using Small = typename std::conditional<GATEUP, Tilings<bf16_t>::GateUpSmall,
                                           Tilings<bf16_t>::BigSmall>::type;
 };
-// fp32 (config 1: T = 1024, H = 384, I = 1024): 64-column tiles give the
-// N = H GEMMs 96 workgroups instead of the 48 that 128-column tiles leave for
-// 256 CUs (config 1 step 0.48 -> 0.37 ms, same bits); for the router and the
-// weight-gradient pair they measured no faster.  64-row tiles for the
-// row-grouped GEMMs double the workgroups again (~256 rows per expert: gate/up
-// input gradient 86 -> 55 us, down forward 40 -> 27 us, step 0.321 -> 0.297
-// ms); the weight-gradient pair on 64 x 128 tiles as well (gate/up weight
-// gradient 55 -> 48 us, step 0.300 -> 0.292 ms), and the router GEMMs and the
-// input gradient dx (dx 16.8 -> 11.8 us, step 0.292 -> 0.288 ms).
+// fp32 (config 1: T = 1024, H = 384, I = 1024): 64 x 64 tiles for the expert
+// GEMMs.  Its ~256-row experts then give the N = H launches 240 workgroups; the
+// router GEMMs and the input gradient dx keep 64 x 128.  A 32 x 32 block per
+// wave is one accumulator, so what fills the matrix cores is several workgroups
+// to a CU: the gate/up forward and the weight-gradient pair, with three
+// operands, run 16-deep k-tiles in three stages (36 KB of LDS, four workgroups
+// to a CU, instead of 48 KB and three with 32-deep ones in two).  Launches
+// alone, 32-deep -> 16-deep: gate/up forward of 12 experts of 500 rows (H = 776,
+// I = 1368) 278 -> 240 us (106 TFLOP/s), 16 of 512 (2048, 1408) 802 -> 745 (127);
+// pair of weight gradients, 64 x 128 tiles -> these: config 1 41 -> 33 us, 12
+// experts 251 -> 220 (116 TFLOP/s), one of 1999 rows 128 -> 70, 16 of 512 704 ->
+// 715.  The two-operand GEMMs (32 KB) measured no faster on 16-deep tiles, and
+// 128 x 64, 64 x 128 and 128 x 128 tiles only from some 4000 rows per expert on
+// (128 x 64 3-6 %), at twice the time where there are few.
 constexpr int kF32RowTile = 64;
 template <> struct Tilings<float> {
   using Router = Tiling<float, 64, 128, 32>;
   using RouterDx = Router;
   using RouterNarrow = Router;
-  using GateUp = Tiling<float, kF32RowTile, 64, 32>;
+  using GateUp = Tiling<float, kF32RowTile, 64, 16, 2, 3>;
   using Big = Tiling<float, kF32RowTile, 64, 32>;
-  using WgradPair = Tiling<float, 64, 128, 32>;
+  using WgradPair = Tiling<float, 64, 64, 16, 2, 3>;
 };
 
 // Row-grouped problems: groups split the M dimension (permuted token rows).
@@ -1619,12 +1624,11 @@ __global__ __launch_bounds__(C::THREADS) void k_gateup_dgrad(const T* __restrict
 template <typename T, int NA>
 using WgradTiling = typename std::conditional<NA == 2, typename Tilings<T>::WgradPair,
                                               typename Tilings<T>::Big>::type;
-template <typename T, int NA, bool GROUPED>
+template <typename T, int NA, bool GROUPED, class C>
 MOE_DEV void wgrad_tile(T* smem, int blk, const T* __restrict__ P0, const T* __restrict__ P1,
                         int64_t ldp, const T* __restrict__ Q, int64_t ldq, const KGroups& groups,
                         int M, int N, float alpha, T* const* out0_tab, T* out0_one,
                         T* const* out1_tab, T* out1_one, float* __restrict__ partial) {
-  using C = WgradTiling<T, NA>;
   int grp, split, krow0, K, m0, n0;
   if (!resolve_k(groups, blk, M, N, C::BM, C::BN, grp, split, krow0, K, m0, n0)) return;
   OpDesc<T> a[NA];
@@ -1693,15 +1697,14 @@ MOE_DEV void wgrad_tile(T* smem, int blk, const T* __restrict__ P0, const T* __r
 // dealt over all XCDs instead (skewed counts), tiles of very different K
 // would land unevenly on a static schedule, and the hardware's dispatch
 // balances them better.
-template <typename T, int NA, bool GROUPED>
-__global__ __launch_bounds__((WgradTiling<T, NA>::THREADS)) void k_wgrad(const T* __restrict__ P0, const T* __restrict__ P1,
+template <typename T, int NA, bool GROUPED, class C = WgradTiling<T, NA>>
+__global__ __launch_bounds__(C::THREADS) void k_wgrad(const T* __restrict__ P0, const T* __restrict__ P1,
                                                int64_t ldp, const T* __restrict__ Q, int64_t ldq,
                                                KGroups groups, int M, int N, float alpha,
                                                T* const* out0_tab, T* out0_one,
                                                T* const* out1_tab, T* out1_one,
                                                float* __restrict__ partial, int vblocks,
                                                int slots) {
-  using C = WgradTiling<T, NA>;
   __shared__ __align__(16) T smem[kernel_smem_elems<C, T, NA, 1, NA>()];
   // a grid of `slots` blocks (the host expected whole experts per XCD) runs
   // persistent whatever the flag says; a full grid only when the flag is set
@@ -1709,12 +1712,12 @@ __global__ __launch_bounds__((WgradTiling<T, NA>::THREADS)) void k_wgrad(const T
   const bool persist =
       slots > 0 && (reduced || (groups.xcd_order && groups.xcd_order[groups.G]));
   if (!persist) {
-    wgrad_tile<T, NA, GROUPED>(smem, (int)blockIdx.x, P0, P1, ldp, Q, ldq, groups, M, N, alpha,
+    wgrad_tile<T, NA, GROUPED, C>(smem, (int)blockIdx.x, P0, P1, ldp, Q, ldq, groups, M, N, alpha,
                                out0_tab, out0_one, out1_tab, out1_one, partial);
     return;
   }
   for (int vb = (int)blockIdx.x; blockIdx.x < (unsigned)slots && vb < vblocks; vb += slots) {
-    wgrad_tile<T, NA, GROUPED>(smem, vb, P0, P1, ldp, Q, ldq, groups, M, N, alpha, out0_tab,
+    wgrad_tile<T, NA, GROUPED, C>(smem, vb, P0, P1, ldp, Q, ldq, groups, M, N, alpha, out0_tab,
                                out0_one, out1_tab, out1_one, partial);
     __syncthreads();  // the next tile's loads overwrite the epilogue's LDS
   }

@@ -91,3 +91,23 @@ def test_full_tiles_over_many_experts(T, H, I):
     assert ((counts > 256) & (tails > 64) & (tails <= 128)).any(), counts
     assert (tails > 192).any(), counts
     _check(case, g, o, 1e-2)
+
+
+@pytest.mark.parametrize("spec", [
+    # one column block, one k-tile of one token row per wave's fragment
+    dict(T=65, H=8, E=1, k=1, I=8, S=8),
+    # rows, columns and tokens one vector past 64-wide tiles and 16 / 32-deep k-tiles
+    dict(T=131, H=200, E=3, k=2, I=72, S=136),
+    # experts of about one row: k-tiles of the weight gradients nearly empty
+    dict(T=67, H=136, E=64, k=1, I=72, S=0),
+    # a split dense weight gradient whose last chunk is ragged
+    dict(T=1030, H=64, E=4, k=1, I=24, S=72),
+])
+def test_fp32_k_major_tiles(spec):
+    """fp32 input and weight gradients, whose K-major operands are read as they lie in memory
+    (1e-5: the fp32 bar, 32-bit sums of at most 1030 terms)."""
+    case = Case(**spec, w_std=0.1)
+    g = gpu_run(case, d_aux=0.01, d_z=0.001)
+    o = oracle_run(case, g["logits"], d_aux=0.01, d_z=0.001)
+    _routing_equal(g, o)
+    _check(case, g, o, 1e-5)
