@@ -553,7 +553,7 @@ constexpr int kFusedRouterChunkBytes = 256;
 // tokens: the expert histogram of their k choices (group_hist[b][e], an
 // integer LDS histogram) and the column sums of their probabilities
 // (prob_part[b][e], tokens added in order), so that k_scan over the 16-token
-// groups and k_colsum_final finish the counts, offsets and P.
+// groups and the column sums beside it finish the counts, offsets and P.
 template <typename T, int NEB>
 __global__ __launch_bounds__(64 * kRouterWaves) __attribute__((amdgpu_waves_per_eu(8))) void k_router_route(
     const T* __restrict__ x, const T* __restrict__ wr, const float* __restrict__ bias,
@@ -691,87 +691,102 @@ __global__ __launch_bounds__(1024) void k_reduce_route(
 }
 
 // ------------------------------------------------------------------ column sums
-// part[rb, e] = sum over rows [rb*64, rb*64+64) of a[t, e], fixed order.
-__global__ __launch_bounds__(256) void k_colsum_partial(const float* __restrict__ a, int Tn, int E,
-                                                        float* __restrict__ part) {
-  __shared__ float red[4][64];
-  const int c = threadIdx.x & 63, r = threadIdx.x >> 6;
-  const int e = blockIdx.x * 64 + c;
-  const int t0 = blockIdx.y * 64;
+// part[rb, e] = sum over rows [rb*64, rb*64+64) of a[t, e], fixed order: unit u
+// (ceil(E / 64) units to a row block, then the next one) by 256 threads, tid of
+// them, with their own red.  Every thread of the workgroup must call it.
+MOE_DEV void colsum_unit(const float* __restrict__ a, int Tn, int E, float* __restrict__ part,
+                         int u, int tid, float (&red)[4][64]) {
+  const int neb = (E + 63) / 64;
+  const int c = tid & 63, r = tid >> 6;
+  const int rb = u / neb, e = (u - rb * neb) * 64 + c;
+  const int t0 = rb * 64;
   float s = 0.0f;
   if (e < E)
     for (int t = t0 + r; t < min(t0 + 64, Tn); t += 4) s += a[(int64_t)t * E + e];
   red[r][c] = s;
   __syncthreads();
-  if (r == 0 && e < E)
-    part[(int64_t)blockIdx.y * E + e] = ((red[0][c] + red[1][c]) + red[2][c]) + red[3][c];
+  if (r == 0 && e < E && t0 < Tn)
+    part[(int64_t)rb * E + e] = ((red[0][c] + red[1][c]) + red[2][c]) + red[3][c];
+}
+__global__ __launch_bounds__(256) void k_colsum_partial(const float* __restrict__ a, int Tn, int E,
+                                                        float* __restrict__ part) {
+  __shared__ float red[4][64];
+  colsum_unit(a, Tn, E, part, (int)blockIdx.x, threadIdx.x, red);
 }
 
-// out[e] = scale * sum_rb part[rb, e]: four running sums over rb = 4 i + j
-// (independent loads stay in flight), added in the fixed order j = 0..3.
-__global__ void k_colsum_final(const float* __restrict__ part, int nrb, int E, float scale,
-                               float* __restrict__ out) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= E) return;
+// scale * sum_rb part[rb, e]: four running sums over rb = 4 i + j (independent
+// loads stay in flight), added in the fixed order j = 0..3.
+MOE_DEV float colsum_final(const float* __restrict__ part, int nrb, int E, int e, float scale) {
   float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   int rb = 0;
   for (; rb + 4 <= nrb; rb += 4)
 #pragma unroll
     for (int j = 0; j < 4; ++j) s[j] += part[(int64_t)(rb + j) * E + e];
   for (; rb < nrb; ++rb) s[rb & 3] += part[(int64_t)rb * E + e];
-  out[e] = (((s[0] + s[1]) + s[2]) + s[3]) * scale;
+  return (((s[0] + s[1]) + s[2]) + s[3]) * scale;
+}
+__global__ void k_colsum_final(const float* __restrict__ part, int nrb, int E, float scale,
+                               float* __restrict__ out) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < E) out[e] = colsum_final(part, nrb, E, e, scale);
 }
 
-// aux = E (c_sw sum_e f_e P_e + c_sq sum_e P_e^2), z = mean_t lse_t^2.
-// counts == nullptr: the expert counts are built here from the top-k indices
-// (integer LDS histogram, E <= 1024), so the kernel can run beside the
-// dispatch instead of after it.
-__global__ __launch_bounds__(256) void k_losses(const float* __restrict__ P,
-                                                const int* __restrict__ counts,
-                                                const int* __restrict__ idx,
-                                                const float* __restrict__ lse, int Tn, int E,
-                                                int k, float c_sw, float c_sq,
-                                                float* __restrict__ aux, float* __restrict__ z) {
-  __shared__ float r_sw[256], r_sq[256], r_z[256];
-  __shared__ int hist[1024];
-  const int tid = threadIdx.x;
-  if (!counts) {
-    for (int e = tid; e < E; e += 256) hist[e] = 0;
-    __syncthreads();
-    const int64_t n = (int64_t)Tn * k;
-    for (int64_t i = tid; i < n; i += 256) {
-      const int e = idx[i];
-      if ((unsigned)e < (unsigned)E) atomicAdd(&hist[e], 1);
-    }
-    __syncthreads();
+// aux = E (c_sw sum_e f_e P_e + c_sq sum_e P_e^2) and z = mean_t lse_t^2 from the
+// 256 partial sums of each in r (a binary tree over lane distances 128, 64, ...
+// 1), by one wave.
+MOE_DEV void write_losses(const float (&r)[3][256], int E, int Tn, float c_sw, float c_sq,
+                          float* __restrict__ aux, float* __restrict__ z) {
+  const int lane = threadIdx.x & 63;
+  float v[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+    v[j] = wave_sum((r[j][lane] + r[j][lane + 128]) + (r[j][lane + 64] + r[j][lane + 192]));
+  if (lane == 0) {
+    if (aux) *aux = (float)E * (c_sw * v[0] + c_sq * v[1]);
+    if (z) *z = v[2] / (float)Tn;
   }
-  const float inv_tk = 1.0f / ((float)Tn * (float)k);
-  float sw = 0.0f, sq = 0.0f, zz = 0.0f;
-  for (int e = tid; e < E; e += 256) {
-    const float p = P[e];
-    sw += ((float)(counts ? counts[e] : hist[e]) * inv_tk) * p;
+}
+
+// The forward's statistics of a batch: the mean probabilities P from their
+// column partials and the losses, by one workgroup of 256 threads.  It rides
+// the combine (k_combine_fwd's first block): everything it reads is long done
+// and only the backward and the caller read what it writes.
+struct LossArgs {
+  const float* part;  // column partials of the probabilities (null: no statistics)
+  int nrb;            // rows of part
+  const int* counts;
+  const float* lse;
+  int Tn, E, k;
+  float c_sw, c_sq;
+  float *P, *aux, *z;
+};
+MOE_DEV void loss_stats(const LossArgs& a) {
+  __shared__ float r[3][256];
+  const int tid = threadIdx.x;
+  const float scale = 1.0f / (float)a.Tn, inv_tk = 1.0f / ((float)a.Tn * (float)a.k);
+  float sw = 0.0f, sq = 0.0f;
+  for (int e = tid; e < a.E; e += 256) {
+    const float p = colsum_final(a.part, a.nrb, a.E, e, scale);
+    a.P[e] = p;
+    sw += ((float)a.counts[e] * inv_tk) * p;
     sq += p * p;
   }
-  {
-    float zp[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // independent loads in flight
-    int t = tid, j = 0;
-    for (; t < Tn; t += 256, j = (j + 1) & 3) zp[j] += lse[t] * lse[t];
-    zz = ((zp[0] + zp[1]) + zp[2]) + zp[3];
+  // lse^2 of every 256th token, the i-th of them to running sum i mod 4; 16
+  // loads in flight
+  float zp[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int t0 = tid; t0 < a.Tn; t0 += 16 * 256) {
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = t0 + 256 * i < a.Tn ? a.lse[t0 + 256 * i] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (t0 + 256 * i < a.Tn) zp[i & 3] += v[i] * v[i];
   }
-  r_sw[tid] = sw; r_sq[tid] = sq; r_z[tid] = zz;
+  r[0][tid] = sw;
+  r[1][tid] = sq;
+  r[2][tid] = ((zp[0] + zp[1]) + zp[2]) + zp[3];
   __syncthreads();
-  for (int o = 128; o >= 1; o >>= 1) {
-    if (tid < o) {
-      r_sw[tid] += r_sw[tid + o];
-      r_sq[tid] += r_sq[tid + o];
-      r_z[tid] += r_z[tid + o];
-    }
-    __syncthreads();
-  }
-  if (tid == 0) {
-    if (aux) *aux = (float)E * (c_sw * r_sw[0] + c_sq * r_sq[0]);
-    if (z) *z = r_z[0] / (float)Tn;
-  }
+  if (tid < 64) write_losses(r, a.E, a.Tn, a.c_sw, a.c_sq, a.aux, a.z);
 }
 
 // ------------------------------------------------------------------ dispatch
@@ -807,21 +822,16 @@ constexpr int prefix_slot(int bm) {
 // others take none.
 constexpr int tall_rows_for(int bm) { return bm == 256 ? bm / 4 : 0; }
 
-// Inclusive prefix sums across the 64 lanes of a wave of N values at once:
-// each step issues the N shuffles before adding, so the N scans wait for one
-// LDS round trip per step instead of N.
-template <int N>
-MOE_DEV void wave_incl_scans(int (&v)[N]) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    int t[N];
-#pragma unroll
-    for (int j = 0; j < N; ++j) t[j] = __shfl_up(v[j], o, 64);
-#pragma unroll
-    for (int j = 0; j < N; ++j)
-      if (lane >= o) v[j] += t[j];
-  }
+// Inclusive prefix sum across the 64 lanes of a wave: DPP row shifts inside the
+// rows of 16 lanes, then the row totals broadcast to the rows above.
+MOE_DEV int wave_incl_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15, rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31, rows 2 and 3
+  return v;
 }
 
 // With cnt[e] (LDS, e < E <= 1024) in place, a block of 1024 threads writes
@@ -849,9 +859,8 @@ MOE_DEV void scan_counts(const int* cnt, int E, int* __restrict__ offsets,
            : kind == 1 ? c / bm + (r > bm / 2 ? 1 : 0)
                        : (tail && r <= bm / 2 ? 1 : 0);
     }
-    incl[j] = v[j];
+    incl[j] = wave_incl_scan(v[j]);
   }
-  wave_incl_scans(incl);
 #pragma unroll
   for (int j = 0; j < kScanCount; ++j)
     if (lane == 63) wsum[j * 16 + wave] = incl[j];
@@ -881,29 +890,25 @@ MOE_DEV void scan_counts(const int* cnt, int E, int* __restrict__ offsets,
 // round of loads, all in flight); longer ones are read twice, eight loads in
 // flight.  Integer arithmetic only.
 constexpr int kScanRegChunk = 64;
-__global__ __launch_bounds__(1024) void k_scan(const int* __restrict__ block_hist, int nb, int E,
-                                               int* __restrict__ block_base,
-                                               int* __restrict__ counts,
-                                               int* __restrict__ offsets,
-                                               int* __restrict__ tile_prefix) {
-  __shared__ int cnt[1024], offs[1024], part[1024];
-  __shared__ int wsum[16 * kScanCount];
+template <int CH>  // histogram entries of a chunk kept in registers (0: read twice)
+MOE_DEV void scan_histograms(const int* __restrict__ block_hist, int nb, int E,
+                             int* __restrict__ block_base, int* __restrict__ counts,
+                             int* __restrict__ offsets, int* __restrict__ tile_prefix, int chunk,
+                             int* cnt, int* offs, int (*part)[1024], int* wsum) {
   const int tid = threadIdx.x;
   const int G = 1024 / E;            // threads per expert
   const int e = tid % E, g = tid / E;
   const bool act = g < G;
-  const int chunk = (nb + G - 1) / G;
   const int b0 = act ? g * chunk : 0, b1 = act ? min(nb, b0 + chunk) : 0;
   const int n = b1 - b0;
-  const bool in_regs = chunk <= kScanRegChunk;  // the same in every thread
-  int c[kScanRegChunk];
+  int c[CH > 0 ? CH : 1];
   int sum = 0;
   constexpr int U = 8;
-  if (in_regs) {
+  if constexpr (CH > 0) {
 #pragma unroll
-    for (int u = 0; u < kScanRegChunk; ++u) c[u] = u < n ? block_hist[(int64_t)(b0 + u) * E + e] : 0;
+    for (int u = 0; u < CH; ++u) c[u] = u < n ? block_hist[(int64_t)(b0 + u) * E + e] : 0;
 #pragma unroll
-    for (int u = 0; u < kScanRegChunk; ++u) sum += c[u];
+    for (int u = 0; u < CH; ++u) sum += c[u];
   } else {
     int b = b0;
     for (; b + U <= b1; b += U) {
@@ -915,27 +920,29 @@ __global__ __launch_bounds__(1024) void k_scan(const int* __restrict__ block_his
     }
     for (; b < b1; ++b) sum += block_hist[(int64_t)b * E + e];
   }
-  // inclusive scan of the chunk sums over g, per expert
-  part[tid] = act ? sum : 0;
+  // inclusive scan of the chunk sums over g, per expert (two buffers, one
+  // barrier a step)
+  int cur = 0, mine = act ? sum : 0;
+  part[0][tid] = mine;
   __syncthreads();
   for (int d = 1; d < G; d <<= 1) {
-    const int v = act && g >= d ? part[tid - d * E] : 0;
-    __syncthreads();
-    if (act) part[tid] += v;
+    if (act && g >= d) mine += part[cur][tid - d * E];
+    cur ^= 1;
+    part[cur][tid] = mine;
     __syncthreads();
   }
   if (tid < E) {
-    const int total = part[(G - 1) * E + tid];
+    const int total = part[cur][(G - 1) * E + tid];
     cnt[tid] = total;
     counts[tid] = total;
   }
   __syncthreads();
   scan_counts(cnt, E, offsets, tile_prefix, offs, wsum);
   if (!act) return;
-  int run = offs[e] + part[tid] - sum;
-  if (in_regs) {
+  int run = offs[e] + mine - sum;
+  if constexpr (CH > 0) {
 #pragma unroll
-    for (int u = 0; u < kScanRegChunk; ++u)
+    for (int u = 0; u < CH; ++u)
       if (u < n) {
         block_base[(int64_t)(b0 + u) * E + e] = run;
         run += c[u];
@@ -960,6 +967,46 @@ __global__ __launch_bounds__(1024) void k_scan(const int* __restrict__ block_his
   }
 }
 
+// Block 0 scans; the blocks after it (four units each) sum the probabilities'
+// columns (col [col_rows, E]: the router groups' sums, or the probabilities)
+// into col_part.  With P and the losses in the combine's first block a forward
+// needs no second stream for its statistics: three launches and four event calls
+// (about 30 us of host time, and the wait at the end) gone.  Together with the
+// chunk in 8 registers where that holds it and the DPP prefix sums (T = 200, E =
+// 16 forward 120 -> 102 us; T = 300, E = 500 317 -> 296; T = 1500, E = 64 368 ->
+// 358; fp32 training step of T = 1024, E = 8 256 -> 242).
+__global__ __launch_bounds__(1024) void k_scan(const int* __restrict__ block_hist, int nb, int E,
+                                               int* __restrict__ block_base,
+                                               int* __restrict__ counts,
+                                               int* __restrict__ offsets,
+                                               int* __restrict__ tile_prefix,
+                                               const float* __restrict__ col, int col_rows,
+                                               float* __restrict__ col_part) {
+  __shared__ int cnt[1024], offs[1024], part[2][1024];
+  __shared__ int wsum[16 * kScanCount];
+  if (blockIdx.x > 0) {
+    auto* red = reinterpret_cast<float(*)[4][64]>(&part[0][0]);
+    const int sub = threadIdx.x >> 8;
+    colsum_unit(col, col_rows, E, col_part, ((int)blockIdx.x - 1) * 4 + sub, threadIdx.x & 255,
+                red[sub]);
+    return;
+  }
+  const int G = 1024 / E, chunk = (nb + G - 1) / G;
+  if (chunk <= 8)
+    scan_histograms<8>(block_hist, nb, E, block_base, counts, offsets, tile_prefix, chunk, cnt,
+                       offs, part, wsum);
+  else if (chunk <= kScanRegChunk)
+    scan_histograms<kScanRegChunk>(block_hist, nb, E, block_base, counts, offsets, tile_prefix,
+                                   chunk, cnt, offs, part, wsum);
+  else
+    scan_histograms<0>(block_hist, nb, E, block_base, counts, offsets, tile_prefix, chunk, cnt,
+                       offs, part, wsum);
+}
+// Blocks of a k_scan launch that also sums `rows` rows of E columns.
+inline int scan_grid(int rows, int E) {
+  const int units = ((rows + 63) / 64) * ((E + 63) / 64);
+  return 1 + (units + 3) / 4;
+}
 
 // Stable scatter: position of assignment (t, j) = offset of its expert +
 // number of earlier tokens (same expert) before it.  Inside a wave, the lanes
@@ -1348,7 +1395,8 @@ __global__ __launch_bounds__(C::THREADS) void k_down_fwd(const T* __restrict__ A
 // ------------------------------------------------------------------ combine
 // out[t] = sum_j w[t, j] * Y[inv_perm[t, j]] (+ s * Ys[t]) (+ resid[t]), added in
 // that order in fp32 and rounded once (inv_perm == nullptr: Y is token-major,
-// row t * k + j, as the grouped down projection writes it).  One wave per (token, slice of 64
+// row t * k + j, as the grouped down projection writes it).  With stats.part set
+// a first block forms the forward's statistics (loss_stats).  One wave per (token, slice of 64
 // 16-byte vectors of the row); the k expert rows of a slice are all requested
 // before the first one is added.
 constexpr int kCombineSlice = 64;  // 16-byte vectors per wave
@@ -1358,11 +1406,19 @@ __global__ __launch_bounds__(256) void k_combine_fwd(const T* __restrict__ Y,
                                                      const float* __restrict__ w,
                                                      const T* __restrict__ Ys, float s, int Tn,
                                                      int k, int H, const T* __restrict__ resid,
-                                                     T* __restrict__ out) {
+                                                     T* __restrict__ out, LossArgs stats) {
   constexpr int V = Vec16<T>::N;
+  int blk = (int)blockIdx.x;
+  if (stats.part) {
+    if (blk == 0) {
+      loss_stats(stats);
+      return;
+    }
+    --blk;
+  }
   const int nv = H / V;
   const int nsl = (nv + kCombineSlice - 1) / kCombineSlice;
-  const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t wid = (int64_t)blk * 4 + (threadIdx.x >> 6);
   if (wid >= (int64_t)Tn * nsl) return;
   const int t = (int)(wid / nsl), sl = (int)(wid % nsl);
   const int c = sl * kCombineSlice + (threadIdx.x & 63);
@@ -1550,10 +1606,15 @@ __global__ __launch_bounds__(C::THREADS) void k_down_dgrad(const T* __restrict__
 }
 
 // dw[perm[r]] = sum over the 32-column blocks c < nb of dwp[c][r] (c ascending):
-// the combine weights' gradient in (token, slot) order.
+// the combine weights' gradient in (token, slot) order.  Block 0 also writes the
+// has_grad mask when asked for.
 __global__ __launch_bounds__(256) void k_dw_sum(const float* __restrict__ dwp, int nb, int TK,
                                                 const int* __restrict__ perm,
-                                                float* __restrict__ dw) {
+                                                float* __restrict__ dw,
+                                                const int* __restrict__ counts, int E,
+                                                uint8_t* __restrict__ has_grad) {
+  if (has_grad && blockIdx.x == 0)
+    for (int e = threadIdx.x; e < E; e += 256) has_grad[e] = counts[e] > 0 ? 1 : 0;
   const int r = blockIdx.x * 256 + threadIdx.x;
   if (r >= TK) return;
   // 16 loads in flight per thread, then added in block order
@@ -1928,11 +1989,6 @@ __global__ __launch_bounds__(256) void k_router_dgrad(const T* __restrict__ dl, 
       store8(dx + (int64_t)(row0 + r) * H + n, v);
     }
   }
-}
-
-__global__ void k_has_grad(const int* __restrict__ counts, int E, uint8_t* __restrict__ has_grad) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < E) has_grad[e] = counts[e] > 0 ? 1 : 0;
 }
 
 // Sets n bytes at p to zero: 16-byte stores where p + i is 16-byte aligned
@@ -2355,13 +2411,13 @@ __global__ __launch_bounds__(64 * kFrontWaves) void k_small_front(
 // which do not depend on order), the counts, offsets, tile prefixes, the
 // permutation (an assignment's rank within its expert is the number of earlier
 // tokens in the mask) and the list of touched experts (`slots`, nslots of
-// them, when not null); the mean probabilities in k_colsum_partial's and
-// k_colsum_final's order (four running sums over t mod 4, added in order);
-// and, when aux or z is not null, the losses with k_losses' reduction tree.
+// them, when not null); the mean probabilities in colsum_unit's and
+// colsum_final's order (four running sums over t mod 4, added in order);
+// and, when aux or z is not null, the losses as loss_stats forms them.
 // No expert holds more than 64 rows, so every tile prefix follows from the
 // number of touched experts (a touched expert is one row tile of any height, a
 // half tile where those are counted), and one 32-bit scan carries rows and
-// touched experts (at most 1024 each).  One launch instead of three (k_route, a dispatch, k_losses), whose
+// touched experts (at most 1024 each).  One launch instead of three (routing, dispatch, losses), whose
 // probabilities, indices and log-sum-exps stay in LDS.
 //
 // The other blocks run the shared expert's down projection beside it (its
@@ -2429,9 +2485,8 @@ __global__ __launch_bounds__(1024) void k_small_route(
   // counts and the packed prefix sum, one expert per thread
   const int c = tid < E ? __popc(u.s.tmask[tid][0]) + __popc(u.s.tmask[tid][1]) : 0;
   const int mine = c | (c > 0 ? 1 << 16 : 0);
-  int incl[1] = {mine};
-  wave_incl_scans(incl);
-  if (lane == 63) u.s.wsum[wave] = incl[0];
+  const int incl = wave_incl_scan(mine);
+  if (lane == 63) u.s.wsum[wave] = incl;
   __syncthreads();
   int base = 0, total = 0;
 #pragma unroll
@@ -2442,7 +2497,7 @@ __global__ __launch_bounds__(1024) void k_small_route(
   }
   {
     const bool last = tid == E;  // writes the totals (E <= 1023; else thread 1023 does)
-    const int ex = last ? total : base + incl[0] - mine;
+    const int ex = last ? total : base + incl - mine;
     auto put = [&](int at, int q) {
       offsets[at] = q & 0xffff;
 #pragma unroll
@@ -2482,7 +2537,7 @@ __global__ __launch_bounds__(1024) void k_small_route(
     const int first = lane & 60;  // lanes 4e .. 4e + 3 of this wave
     const float r0 = __shfl(r, first, 64), r1 = __shfl(r, first + 1, 64);
     const float r2 = __shfl(r, first + 2, 64), r3 = __shfl(r, first + 3, 64);
-    // k_colsum_final adds this single partial to three zeros: the same value
+    // colsum_final adds this single partial to three zeros: the same value
     if (e < E && q == 0) {
       const float p = (((r0 + r1) + r2) + r3) * scale;
       P[e] = p;
@@ -2514,18 +2569,7 @@ __global__ __launch_bounds__(1024) void k_small_route(
     u.s.r[2][tid] = tid < Tn ? u.s.lse[tid] * u.s.lse[tid] : 0.0f;
   }
   __syncthreads();
-  if (wave == 0) {
-    float v[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const float* r = u.s.r[j];
-      v[j] = wave_sum((r[lane] + r[lane + 128]) + (r[lane + 64] + r[lane + 192]));
-    }
-    if (lane == 0) {
-      if (aux) *aux = (float)E * (c_sw * v[0] + c_sq * v[1]);
-      if (z) *z = v[2] / (float)Tn;
-    }
-  }
+  if (wave == 0) write_losses(u.s.r, E, Tn, c_sw, c_sq, aux, z);
 }
 
 // The list of touched experts alone, from the kept offsets (a recomputing

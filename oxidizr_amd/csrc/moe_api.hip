@@ -273,8 +273,6 @@ struct moe_plan {
   // The backward's routed weight gradients need only dY / dG / dU and the
   // routing state: they run on a third stream, beside the input-gradient
   // GEMMs and the router backward on the call's stream.
-  // In the forward the same stream sums the mean router probabilities (needed
-  // only by the losses) while the call's stream dispatches.
   hipStream_t wgs = nullptr;
   hipEvent_t wfork = nullptr, wmid = nullptr, wjoin = nullptr;
   int overlap = 1;  // 0: serial; 1: shared-expert and weight-gradient streams; 2: shared only
@@ -587,14 +585,12 @@ void launch_small_route(moe_plan* p, hipStream_t s, int T, char* saved, const Sa
 // kernel has written the routing decisions too), losses' P statistics and
 // dispatch.  With `routed` (T > kRouteSmallTokens) the dispatch stops after
 // k_scan: the caller writes perm and inv_perm (k_scatter_groups from the
-// group bases at W.gbase).  pjoin != null: the mean probabilities P may be
-// summed on the plan's weight-gradient stream, forked through *pjoin; the
-// caller joins it before reading P.  Up to kRouteSmallTokens tokens everything
-// is one launch (k_small_route, with `extra`).
+// group bases at W.gbase).  The probabilities' column partials ride k_scan; P
+// itself and the losses ride the combine (loss_args).  Up to kRouteSmallTokens
+// tokens everything is one launch (k_small_route, with `extra`).
 template <typename D>
 moe_status run_routing(moe_plan* p, hipStream_t s, int64_t T64, char* saved, char* ws,
-                       const SavedLayout& L, const WsLayout& W, SideJoin* pjoin,
-                       bool routed = false, const SmallExtra& extra = {}) {
+                       const SavedLayout& L, const WsLayout& W, bool routed = false, const SmallExtra& extra = {}) {
   const moe_config& c = p->cfg;
   const int T = (int)T64, E = c.num_experts, k = c.experts_per_tok;
   float* logits = (float*)(saved + L.f[MOE_SAVED_LOGITS]);
@@ -606,7 +602,6 @@ moe_status run_routing(moe_plan* p, hipStream_t s, int64_t T64, char* saved, cha
   int* offsets = (int*)(saved + L.f[MOE_SAVED_OFFSETS]);
   int* perm = (int*)(saved + L.f[MOE_SAVED_PERM]);
   int* inv = (int*)(saved + L.f[MOE_SAVED_INV_PERM]);
-  float* P = (float*)(saved + L.f[MOE_SAVED_MEAN_PROB]);
   int* tprefix = (int*)(saved + L.tile_prefix);
   if (T <= kRouteSmallTokens) {
     StageTimer st(p, s, MOE_STAGE_ROUTE);
@@ -636,38 +631,22 @@ moe_status run_routing(moe_plan* p, hipStream_t s, int64_t T64, char* saved, cha
       default: launch_route<16>(s, grid, logits, T, E, k, tau, c.norm_topk_prob, probs, lse, idx, w); break;
     }
     LAUNCH_CHECK();
-    const hipStream_t ps = pjoin ? p->wgrad_stream(s) : s;
-    if (pjoin) HIP_TRY(pjoin->fork(s, ps, p->wfork, p->wjoin));
-    if (routed) {  // P from the fused router's per-group sums, in two fixed-order levels
-      const int ng = route_groups(T), nrb = colsum_rows(T, true);
-      float* part = (float*)(ws + W.colpart);
-      hipLaunchKernelGGL(k_colsum_partial, dim3(ceil_div(E, 64), nrb), dim3(256), 0, ps,
-                         (const float*)(ws + W.gpart), ng, E, part);
-      hipLaunchKernelGGL(k_colsum_final, dim3(ceil_div(E, 256)), dim3(256), 0, ps, part, nrb, E,
-                         1.0f / (float)T, P);
-    } else {
-      const int nrb = colsum_rows(T, false);
-      float* part = (float*)(ws + W.colpart);
-      hipLaunchKernelGGL(k_colsum_partial, dim3(ceil_div(E, 64), nrb), dim3(256), 0, ps, probs,
-                         T, E, part);
-      hipLaunchKernelGGL(k_colsum_final, dim3(ceil_div(E, 256)), dim3(256), 0, ps, part, nrb, E,
-                         1.0f / (float)T, P);
-    }
-    LAUNCH_CHECK();
   }
   {
     StageTimer st(p, s, MOE_STAGE_DISPATCH);
     if (routed) {  // the fused router counted its 16-token groups' choices
       const int ng = route_groups(T);
       int* gb = (int*)(ws + W.gbase);
-      hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, (const int*)(ws + W.ghist), ng, E, gb,
-                         counts, offsets, tprefix);
+      hipLaunchKernelGGL(k_scan, dim3(scan_grid(ng, E)), dim3(1024), 0, s,
+                         (const int*)(ws + W.ghist), ng, E, gb, counts, offsets, tprefix,
+                         (const float*)(ws + W.gpart), ng, (float*)(ws + W.colpart));
     } else {
       const int nb = hist_blocks(T);
       int* bh = (int*)(ws + W.block_hist);
       int* bb = (int*)(ws + W.block_base);
       hipLaunchKernelGGL(k_hist, dim3(nb), dim3(256), sizeof(int) * E, s, idx, T, k, E, bh);
-      hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, bh, nb, E, bb, counts, offsets, tprefix);
+      hipLaunchKernelGGL(k_scan, dim3(scan_grid(T, E)), dim3(1024), 0, s, bh, nb, E, bb, counts,
+                         offsets, tprefix, probs, T, (float*)(ws + W.colpart));
       hipLaunchKernelGGL(k_scatter, dim3(nb), dim3(256), sizeof(int) * 16 * E, s, idx, T, k, E,
                          bb, perm, inv);
     }
@@ -1053,7 +1032,7 @@ moe_status forward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* x,
   // small bf16 batch runs it beside the router on the call's own stream.
   const bool skinny = std::is_same<D, bf16_t>::value && T <= kSkinnyMaxTokens;
   D* sY = S > 0 ? (D*)(ws + W.sY) : nullptr;
-  SideJoin shared_join, p_join;
+  SideJoin shared_join;
   if (S > 0 && !skinny) {
     const hipStream_t ss = p->shared_stream(s);
     HIP_TRY(shared_join.fork(s, ss, p->fork, p->join));
@@ -1144,18 +1123,8 @@ moe_status forward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* x,
     extra.sd = (const bf16_t*)w->shared_down;
     extra.sY = (bf16_t*)sY;
   }
-  moe_status r = run_routing<D>(p, s, T64, rb, ws, LR, W, &p_join, fused, extra);
+  moe_status r = run_routing<D>(p, s, T64, rb, ws, LR, W, fused, extra);
   if (r != MOE_OK) return r;
-  if (T > kRouteSmallTokens) {  // k_small_route forms a small batch's losses
-    // beside the dispatch when P is summed on the side stream (the kernel
-    // then counts the experts itself), else after the dispatch on s
-    const bool side = p_join.armed;
-    const hipStream_t ls = side ? p_join.side : s;
-    StageTimer tm(p, ls, MOE_STAGE_LOSSES);
-    hipLaunchKernelGGL(k_losses, dim3(1), dim3(256), 0, ls, st.P, side ? nullptr : st.counts,
-                       st.idx, st.lse, T, E, k, c.aux_switch_coef, c.aux_sqprob_coef, aux, z);
-    LAUNCH_CHECK();
-  }
   if ((r = routed_fwd<D>(p, s, T, x, st, true, defer ? (const int*)(ws + W.gbase) : nullptr)) !=
       MOE_OK)
     return r;
@@ -1165,12 +1134,17 @@ moe_status forward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* x,
     const int nsl = ceil_div(H / (16 / (int)sizeof(D)), kCombineSlice);
     // the tiled down projection writes Y token-major; the small-token kernel
     // in expert order
-    hipLaunchKernelGGL(k_combine_fwd<D>, dim3(ceil_div((int64_t)T * nsl, 4)), dim3(256), 0, s,
-                       st.Y, skinny ? st.inv : nullptr,
-                       st.w, sY, c.shared_expert_scale, T, k, H, resid, out);
+    // k_small_route has formed a small batch's statistics
+    LossArgs stats{};
+    if (T > kRouteSmallTokens)
+      stats = LossArgs{(const float*)(ws + W.colpart), colsum_rows(T, fused), st.counts, st.lse, T,
+                       E, k, c.aux_switch_coef, c.aux_sqprob_coef, st.P, aux, z};
+    hipLaunchKernelGGL(k_combine_fwd<D>,
+                       dim3(ceil_div((int64_t)T * nsl, 4) + (stats.part ? 1 : 0)), dim3(256), 0, s,
+                       st.Y, skinny ? st.inv : nullptr, st.w, sY, c.shared_expert_scale, T, k, H,
+                       resid, out, stats);
     LAUNCH_CHECK();
   }
-  HIP_TRY(p_join.join());  // P and the losses
   return MOE_OK;
 }
 
@@ -1345,7 +1319,7 @@ moe_status backward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* dout,
     });
     LAUNCH_CHECK();
     hipLaunchKernelGGL(k_dw_sum, dim3(ceil_div(TK, (int64_t)256)), dim3(256), 0, s, dwp,
-                       ceil_div(I, 32), (int)TK, st.perm, dw);
+                       ceil_div(I, 32), (int)TK, st.perm, dw, counts, E, has_grad);
     LAUNCH_CHECK();
   }
   // the gate/up weight gradient's token rows, weighted (its dG_u, dU_u leave
@@ -1402,7 +1376,7 @@ moe_status backward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* dout,
     if (c.has_router_bias && g->router_bias) {
       const int nrb = colsum_rows(T, false);
       float* part = (float*)(ws);  // column partials at workspace offset 0
-      hipLaunchKernelGGL(k_colsum_partial, dim3(ceil_div(E, 64), nrb), dim3(256), 0, s, dl, T, E,
+      hipLaunchKernelGGL(k_colsum_partial, dim3(ceil_div(E, 64) * nrb), dim3(256), 0, s, dl, T, E,
                          part);
       hipLaunchKernelGGL(k_colsum_final, dim3(ceil_div(E, 256)), dim3(256), 0, s, part, nrb, E,
                          1.0f, g->router_bias);
@@ -1425,7 +1399,6 @@ moe_status backward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* dout,
       hipLaunchKernelGGL((k_router_dgrad<D, 8>), grid, dim3(256), 0, s, dlt, Epad, E, wr, T, H, dXp, nullptr, k, topw, dxs, dx);
     else
       hipLaunchKernelGGL((k_router_dgrad<D, 16>), grid, dim3(256), 0, s, dlt, Epad, E, wr, T, H, dXp, nullptr, k, topw, dxs, dx);
-    if (has_grad) hipLaunchKernelGGL(k_has_grad, dim3(ceil_div(E, 256)), dim3(256), 0, s, counts, E, has_grad);
     LAUNCH_CHECK();
   }
   HIP_TRY(wgrad_join.join());
@@ -2027,8 +2000,16 @@ moe_status moe_route_from_logits(moe_plan* p, void* stream, int64_t T, const flo
   HIP_TRY(hipMemcpyAsync(sv + L.f[MOE_SAVED_LOGITS], logits,
                          sizeof(float) * (size_t)T * p->cfg.num_experts, hipMemcpyDeviceToDevice,
                          s));
-  if (p->cfg.dtype == MOE_DTYPE_BF16) return run_routing<bf16_t>(p, s, T, sv, (char*)workspace, L, W, nullptr);
-  return run_routing<float>(p, s, T, sv, (char*)workspace, L, W, nullptr);
+  const moe_status st2 = p->cfg.dtype == MOE_DTYPE_BF16
+                             ? run_routing<bf16_t>(p, s, T, sv, (char*)workspace, L, W)
+                             : run_routing<float>(p, s, T, sv, (char*)workspace, L, W);
+  if (st2 != MOE_OK || T <= kRouteSmallTokens) return st2;
+  const int E = p->cfg.num_experts;  // P, which rides the combine in a forward
+  hipLaunchKernelGGL(k_colsum_final, dim3(ceil_div(E, 256)), dim3(256), 0, s,
+                     (const float*)((char*)workspace + W.colpart), colsum_rows(T, false), E,
+                     1.0f / (float)T, (float*)(sv + L.f[MOE_SAVED_MEAN_PROB]));
+  LAUNCH_CHECK();
+  return MOE_OK;
 }
 
 const char* moe_stage_name(int32_t stage) {

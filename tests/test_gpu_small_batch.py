@@ -63,3 +63,29 @@ def test_topk_of_special_values(T, E, k):
     np.testing.assert_array_equal(f("counts"), counts)
     np.testing.assert_array_equal(f("perm"), perm)
     np.testing.assert_array_equal(f("inv_perm"), inv)
+
+
+@pytest.mark.parametrize("T,E,k", [(65, 1, 1), (64, 70, 3), (1000, 3, 2), (2500, 1000, 4),
+                                   (18000, 1000, 2), (5000, 300, 16)])
+def test_dispatch_and_mean_probabilities_of_given_logits(T, E, k):
+    # k_scan's three chunk sizes (at most 8 and 64 histogram blocks to a thread, more) with
+    # the column sums that ride it; P within 32-bit sums of T terms in rows of 64
+    rng = np.random.default_rng(T + E)
+    logits = rng.normal(size=(T, E)).astype(np.float32)
+    cfg = MoeConfig(hidden_size=8, num_experts=E, experts_per_tok=k, intermediate_size=8,
+                    shared_expert_enabled=False)
+    dev = torch.device("cuda:0")
+    plan = Plan(cfg, torch.float32, dev)
+    saved = plan.route_from_logits(torch.tensor(logits, device=dev))
+    torch.cuda.synchronize()
+    f = lambda n: plan.saved_field(saved, T, n).cpu().numpy()
+    want = np.argsort(-logits, axis=1, kind="stable")[:, :k].astype(np.int32)
+    np.testing.assert_array_equal(f("topk_idx"), want)
+    counts, offsets, perm, inv = mo.dispatch(want, E)
+    np.testing.assert_array_equal(f("counts"), counts)
+    np.testing.assert_array_equal(f("offsets"), offsets)
+    np.testing.assert_array_equal(f("perm"), perm)
+    np.testing.assert_array_equal(f("inv_perm"), inv)
+    p = np.exp(logits.astype(np.float64))
+    p /= p.sum(1, keepdims=True)
+    np.testing.assert_allclose(f("mean_prob"), p.mean(0), rtol=2e-5)
