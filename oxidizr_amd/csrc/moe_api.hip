@@ -1293,8 +1293,12 @@ moe_status backward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* dout,
     LAUNCH_CHECK();
   }
   // whole experts per XCD for the gate/up weight gradient when the experts
-  // split evenly over the XCDs (k_xcd_order decides on the device)
-  int* xorder = E % 8 == 0 ? (int*)(ws + W.xorder) : nullptr;
+  // split evenly over the XCDs (k_xcd_order decides on the device) and average
+  // at least a k-tile of rows: with fewer, the launch is its output stores and
+  // persistent workgroups only serialise them (E = 64, 56 rows each, H = 2048, I
+  // = 1408: step 1033 -> 993 us without; E = 16, 62 rows: 400 -> 393; E = 128, 136
+  // rows: 1663 with, 1682 without)
+  int* xorder = E % 8 == 0 && TK >= 64 * (int64_t)E ? (int*)(ws + W.xorder) : nullptr;
   if (p->xflag_pending && hipEventQuery(p->xflag_ev) == hipSuccess) {
     p->xflag = *p->h_xflag;
     p->xflag_pending = false;
