@@ -2182,6 +2182,9 @@ struct SkinnySlot {
   int r0, rows;
   const bf16_t *gate, *up, *down;
 };
+// The list lies where the layout of a call's activations holds tile prefixes
+// that such a call does not use.
+static_assert(sizeof(SkinnySlot) <= sizeof(int) * kNumTilePrefixes, "E slots in the tile prefixes");
 
 // A skinny workgroup of NW waves: KS waves share the 16 weight rows of one row
 // block and take every KS-th k-chunk of it (partial sums added in wave order),
@@ -2500,9 +2503,11 @@ __global__ __launch_bounds__(1024) void k_small_route(
     const int ex = last ? total : base + incl - mine;
     auto put = [&](int at, int q) {
       offsets[at] = q & 0xffff;
+      if (tile_prefix) {  // null: no tiled kernel follows
 #pragma unroll
-      for (int j = 0; j < kNumTilePrefixes; ++j)
-        tile_prefix[j * (E + 1) + at] = kPrefixKind[j] == 1 ? 0 : q >> 16;
+        for (int j = 0; j < kNumTilePrefixes; ++j)
+          tile_prefix[j * (E + 1) + at] = kPrefixKind[j] == 1 ? 0 : q >> 16;
+      }
     };
     if (tid <= E) put(tid, ex);
     if (E == 1024 && tid == 1023) put(1024, total);

@@ -237,9 +237,6 @@ struct moe_plan {
   void* scratch_ptr = nullptr;  // device address of `scratch` on this plan's device
   // device pointer tables: 0 gate, 1 up, 2 down (weights); 3..5 their grads
   void** d_tab = nullptr;
-  // the touched experts of a small batch (bf16 plans), written by its routing
-  // and read by its expert launches; like the tables, one call at a time
-  SkinnySlot* d_slots = nullptr;
   // Pinned host staging for table uploads: a ring of kTabSlots slots of 6 E
   // pointers.  A slot is refilled only after the copy that last read it has
   // run (its event), so an upload never waits for the stream as a whole.
@@ -548,12 +545,14 @@ void launch_router_route(hipStream_t s, int T, const D* x, const D* wr, const fl
 }
 
 // What k_small_route does beside the routing of a small batch: the losses (when
-// aux or z is not null), the list of touched experts (skinny) and the shared
-// expert's down projection sY = sA Wd^T (S > 0).
+// aux or z is not null), the list of touched experts (slots not null; then the
+// tile prefixes only with `prefixes`) and the shared expert's down projection sY =
+// sA Wd^T (S > 0).
 struct SmallExtra {
   float* aux = nullptr;
   float* z = nullptr;
-  bool skinny = false;
+  SkinnySlot* slots = nullptr;
+  bool prefixes = true;
   int S = 0;
   const bf16_t* sA = nullptr;
   const bf16_t* sd = nullptr;
@@ -576,9 +575,9 @@ void launch_small_route(moe_plan* p, hipStream_t s, int T, char* saved, const Sa
                      c.router_temperature, c.norm_topk_prob, c.aux_switch_coef, c.aux_sqprob_coef,
                      f(MOE_SAVED_PROBS), f(MOE_SAVED_LSE), i(MOE_SAVED_TOPK_IDX),
                      f(MOE_SAVED_TOPK_W), f(MOE_SAVED_MEAN_PROB), i(MOE_SAVED_COUNTS),
-                     i(MOE_SAVED_OFFSETS), (int*)(saved + L.tile_prefix), i(MOE_SAVED_PERM),
+                     i(MOE_SAVED_OFFSETS), x.prefixes ? (int*)(saved + L.tile_prefix) : nullptr, i(MOE_SAVED_PERM),
                      i(MOE_SAVED_INV_PERM), x.aux, x.z, tab, tab + E, tab + 2 * E,
-                     x.skinny ? p->d_slots : nullptr, small_slots(c, T), x.sA, x.sd, x.S, H, x.sY);
+                     x.slots, small_slots(c, T), x.sA, x.sd, x.S, H, x.sY);
 }
 
 // Routing (from logits already in saved, unless `routed`: the fused router
@@ -935,7 +934,7 @@ void with_row_tiling(const int* offsets, const int* tprefix_all, int E, int64_t 
 // then writes perm and inv_perm.
 template <typename D>
 moe_status routed_fwd(moe_plan* p, hipStream_t s, int T, const D* x, const State<D>& st,
-                      bool timed, const int* gbase = nullptr) {
+                      bool timed, const int* gbase = nullptr, const SkinnySlot* slots = nullptr) {
   using CG = typename Tilings<D>::GateUp;
   using CB = typename Tilings<D>::Big;
   const moe_config& c = p->cfg;
@@ -943,7 +942,7 @@ moe_status routed_fwd(moe_plan* p, hipStream_t s, int T, const D* x, const State
   const int64_t TK = (int64_t)T * k;
   auto stage = [&](int id) { return timed ? id : MOE_STAGE_RECOMPUTE; };
   // few tokens: no expert holds more than T rows, stream the weights of the
-  // experts that the routing listed (p->d_slots) instead
+  // experts that the routing listed in `slots` instead
   const bool skinny = std::is_same<D, bf16_t>::value && T <= kSkinnyMaxTokens;
   if (gbase) {  // the dispatch's last launch
     StageTimer tm(p, s, stage(MOE_STAGE_DISPATCH));
@@ -961,7 +960,7 @@ moe_status routed_fwd(moe_plan* p, hipStream_t s, int T, const D* x, const State
       auto go = [&](auto nc) {
         hipLaunchKernelGGL((k_skinny_fwd<true, decltype(nc)::value, KS>),
                            dim3(skinny_grid<KS>(small_slots(c, T), I)), dim3(256), 0, s,
-                           (const bf16_t*)x, st.perm, k, T, p->d_slots, 0, nullptr, nullptr, H, I,
+                           (const bf16_t*)x, st.perm, k, T, slots, 0, nullptr, nullptr, H, I,
                            (bf16_t*)st.G, (bf16_t*)st.U, (bf16_t*)st.A);
       };
       if (T <= 16) go(std::integral_constant<int, 1>());
@@ -984,7 +983,7 @@ moe_status routed_fwd(moe_plan* p, hipStream_t s, int T, const D* x, const State
       auto go = [&](auto nc) {
         hipLaunchKernelGGL((k_skinny_fwd<false, decltype(nc)::value, KS>),
                            dim3(skinny_grid<KS>(small_slots(c, T), H)), dim3(256), 0, s,
-                           (const bf16_t*)st.A, nullptr, 1, 0, p->d_slots, 0, nullptr, nullptr, I,
+                           (const bf16_t*)st.A, nullptr, 1, 0, slots, 0, nullptr, nullptr, I,
                            H, (bf16_t*)st.Y, nullptr, nullptr);
       };
       if (T <= 16) go(std::integral_constant<int, 1>());
@@ -1128,7 +1127,10 @@ moe_status forward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* x,
   extra.aux = aux;
   extra.z = z;
   if (skinny) {
-    extra.skinny = true;
+    // the list of touched experts, in the forward-only state's tile prefixes: no
+    // tiled kernel of this call reads those, and a backward's are in `saved`
+    extra.slots = (SkinnySlot*)(ws + W.infer + LT.tile_prefix);
+    extra.prefixes = train;
     extra.S = S;
     extra.sA = (const bf16_t*)st.sA;
     extra.sd = (const bf16_t*)w->shared_down;
@@ -1136,8 +1138,8 @@ moe_status forward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* x,
   }
   moe_status r = run_routing<D>(p, s, T64, rb, ws, LR, W, fused, extra);
   if (r != MOE_OK) return r;
-  if ((r = routed_fwd<D>(p, s, T, x, st, true, defer ? (const int*)(ws + W.gbase) : nullptr)) !=
-      MOE_OK)
+  if ((r = routed_fwd<D>(p, s, T, x, st, true, defer ? (const int*)(ws + W.gbase) : nullptr,
+                         extra.slots)) != MOE_OK)
     return r;
   HIP_TRY(shared_join.join());
   {
@@ -1269,13 +1271,16 @@ moe_status backward_impl(moe_plan* p, hipStream_t s, int64_t T64, const D* dout,
     if (rs != MOE_OK) return rs;
   }
   if (recompute) {
+    SkinnySlot* slots = nullptr;
     if (std::is_same<D, bf16_t>::value && T <= kSkinnyMaxTokens) {
+      // in the rebuilt activations' tile prefixes (the call's own are in `saved`)
+      slots = (SkinnySlot*)(ab + LA.tile_prefix);
       const bf16_t* const* tab = (const bf16_t* const*)p->d_tab;
       hipLaunchKernelGGL(k_small_slots, dim3(1), dim3(1024), 0, s, offsets, E, tab, tab + E,
-                         tab + 2 * E, p->d_slots, small_slots(c, T));
+                         tab + 2 * E, slots, small_slots(c, T));
       LAUNCH_CHECK();
     }
-    moe_status r = routed_fwd<D>(p, s, T, x, st, false);
+    moe_status r = routed_fwd<D>(p, s, T, x, st, false, nullptr, slots);
     if (r != MOE_OK) return r;
   }
   float* dwp = (float*)(ws + W.dwp);
@@ -1664,8 +1669,6 @@ moe_status moe_plan_create(const moe_config* cfg, int device, moe_plan** out) {
   if (e == hipSuccess)
     e = hipHostMalloc((void**)&p->h_tab, tab_bytes * moe_plan::kTabSlots, hipHostMallocDefault);
   if (e == hipSuccess) e = hipMemset(p->d_tab, 0, tab_bytes);
-  if (e == hipSuccess && cfg->dtype == MOE_DTYPE_BF16)
-    e = hipMalloc((void**)&p->d_slots, sizeof(SkinnySlot) * (size_t)cfg->num_experts);
   for (int i = 0; i < moe_plan::kTabSlots && e == hipSuccess; ++i)
     e = hipEventCreateWithFlags(&p->tab_ev[i], hipEventDisableTiming);
   if (e == hipSuccess && cfg->shared_intermediate > 0) {
@@ -1713,7 +1716,6 @@ moe_status moe_plan_destroy(moe_plan* p) {
     (void)hipEventDestroy(p->tab_ev[i]);
   }
   if (p->d_tab) (void)hipFree(p->d_tab);
-  if (p->d_slots) (void)hipFree(p->d_slots);
   if (p->h_tab) (void)hipHostFree(p->h_tab);
   if (p->xflag_ev) {
     if (p->xflag_pending) (void)hipEventSynchronize(p->xflag_ev);

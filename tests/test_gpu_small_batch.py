@@ -89,3 +89,29 @@ def test_dispatch_and_mean_probabilities_of_given_logits(T, E, k):
     p = np.exp(logits.astype(np.float64))
     p /= p.sum(1, keepdims=True)
     np.testing.assert_allclose(f("mean_prob"), p.mean(0), rtol=2e-5)
+
+
+def test_small_batches_of_one_plan_share_no_scratch():
+    # the list of touched experts lies in the call's own workspace: calls of two batches
+    # whose workspaces differ (one per stream) leave each other's lists alone
+    torch.manual_seed(5)
+    dev = torch.device("cuda:0")
+    H, I, E, k = 256, 136, 32, 2
+    cfg = MoeConfig(hidden_size=H, num_experts=E, experts_per_tok=k, intermediate_size=I,
+                    shared_expert_enabled=False)
+    t = lambda *shape: (torch.randn(*shape, device=dev) * 0.05).to(torch.bfloat16)
+    plan = Plan(cfg, torch.bfloat16, dev)
+    router, tabs = t(E, H), [list(t(E, I, H)), list(t(E, I, H)), list(t(E, H, I))]
+    w, keep = plan.weights_struct(router, *tabs)
+    xs = [torch.randn(T, H, device=dev).to(torch.bfloat16) for T in (3, 61)]
+    want = [plan.forward(x, w, need_grad=False)[0].clone() for x in xs]
+    streams = [torch.cuda.Stream(dev) for _ in xs]
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(20):
+        for i, (x, s) in enumerate(zip(xs, streams)):
+            with torch.cuda.stream(s):
+                got[i].append(plan.forward(x, w, need_grad=False)[0])
+    torch.cuda.synchronize()
+    for i in range(2):
+        assert all(torch.equal(g, want[i]) for g in got[i])
