@@ -375,7 +375,7 @@ def measure(args, config, steps, warmup, extras=True):
         layer_bytes = (n_touched * 3 * H * I * b + E * H * b + 2 * T * H * b + T * E * 4 + TK * 8)
         extra = {"layer_hbm_GBs": round(layer_bytes / (elapsed / steps) / 1e9, 1),
                  "layer_hbm_frac": round(layer_bytes / (elapsed / steps) / 1e9 / PEAK_HBM_GBS, 4)}
-        roof["kernel"] = (f"k_skinny_fwd<true, false> (gate/up weight stream + SwiGLU), "
+        roof["kernel"] = (f"k_skinny_fwd (gate/up weight stream + SwiGLU), "
                           f"{dom_avg_ms:.4f} ms/launch")
     else:
         flops, nbytes = gemm_work[dominant]
