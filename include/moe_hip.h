@@ -238,7 +238,10 @@ moe_status moe_saved_field_range(const moe_plan* plan, int64_t num_tokens, int32
 
 /* Per-stage device timing with HIP events recorded on the call's stream
  * around each stage whose bit (1 << moe_stage) is set in stage_mask; -1 times
- * every stage, 0 (the default) none. */
+ * every stage, 0 (the default) none.  A stage whose work rides another's launch
+ * records nothing: the losses (in the combine), and for at most 64 bf16 tokens
+ * the dispatch (in the routing) and the shared expert (beside the router GEMM
+ * and the routing). */
 typedef enum {
   MOE_STAGE_ROUTER_GEMM = 0, MOE_STAGE_ROUTE, MOE_STAGE_DISPATCH, MOE_STAGE_GATHER,
   MOE_STAGE_GATEUP_FWD, MOE_STAGE_DOWN_FWD, MOE_STAGE_SHARED_FWD, MOE_STAGE_COMBINE_FWD,
@@ -253,7 +256,8 @@ moe_status moe_plan_set_profiling(moe_plan* plan, int32_t stage_mask);
  * the call's stream inside every call), so that independent GEMMs fill each
  * other's partial rounds of work.  on = 0 runs everything on the call's
  * stream instead (serial order, for per-kernel measurements); on = 2 uses the
- * second stream only; on = 1 is the default.  Results are bitwise the same
+ * second stream only; on = 1 is the default.  The forward of at most 64 bf16
+ * tokens runs on the call's stream alone.  Results are bitwise the same
  * every way.  No reference counterpart (scheduling knob of this
  * implementation). */
 moe_status moe_plan_set_shared_overlap(moe_plan* plan, int32_t on);
