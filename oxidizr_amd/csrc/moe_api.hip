@@ -197,17 +197,33 @@ SplitPlan plan_split(int M, int N, int K) {
   return {ceil_div(K, chunk), chunk};
 }
 
+// The split of one dense weight gradient (NA outputs of M x N over T tokens).
+// It also decides how many terms one running fp32 sum holds.  The fp32 pair runs
+// 64 x 64 tiles of 16-deep k-tiles, several to a CU, and is planned as 64 x 128
+// tiles of 32-deep ones: the cost model has one workgroup to a CU, and on the
+// launch's own tile it splits less (a tenth of the shapes with M and N up to some
+// thousands).  M = 680, N = 776, T = 1999: 1 chunk instead of 3, and gradients
+// 7.9e-7 off a 64-bit sum instead of 4.6e-7.
+template <typename D, int NA>
+SplitPlan plan_dense_wgrad(int M, int N, int T) {
+  using C = WgradTiling<D, NA>;
+  using P = typename std::conditional<std::is_same<D, float>::value && NA == 2,
+                                      Tiling<float, 64, 128, 32>, C>::type;
+  static_assert(P::BK % C::BK == 0, "chunks are whole k-tiles of the launch");
+  return plan_split<P>(M, N, T);
+}
+
 // fp32 partial-tile bytes of one dense weight gradient (NA outputs of M x N
 // over T tokens) as launch_dense_wgrad splits it: 0 when it runs unsplit.
 template <typename D, int NA>
 size_t dense_wgrad_partial_bytes(int M, int N, int T) {
-  const SplitPlan sp = plan_split<WgradTiling<D, NA>>(M, N, T);
+  const SplitPlan sp = plan_dense_wgrad<D, NA>(M, N, T);
   return sp.nsplit > 1 ? (size_t)NA * sp.nsplit * (size_t)M * N * 4 : 0;
 }
 
 // fp32 partial-tile bytes of the largest dense weight gradient of one backward:
 // the router's, or the shared expert's (they run concurrently, on separate
-// buffers).  Planned with the tilings the launches use (WgradTiling), so the
+// buffers).  Planned with the launches' own plan_dense_wgrad, so the
 // split counts agree; launch_dense_wgrad also refuses a split that would not
 // fit.
 template <typename D>
@@ -669,7 +685,7 @@ moe_status launch_dense_wgrad(hipStream_t s, const D* P0, const D* P1, int64_t l
                               int64_t ldq, int T, int M, int N, float alpha, D* o0, D* o1,
                               float* partial, size_t partial_bytes) {
   using C = WgradTiling<D, NA>;
-  const SplitPlan sp = plan_split<C>(M, N, T);
+  const SplitPlan sp = plan_dense_wgrad<D, NA>(M, N, T);
   if (sp.nsplit > 1) {
     const size_t need = dense_wgrad_partial_bytes<D, NA>(M, N, T);
     if (need > partial_bytes)

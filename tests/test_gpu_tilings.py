@@ -6,7 +6,7 @@ import math
 import numpy as np
 import pytest
 
-from tests.gpu_helpers import Case, gpu_run, oracle_run
+from tests.gpu_helpers import Case, gpu_run, oracle_run, rel
 from tests.test_gpu_parity import _check, _routing_equal
 
 pytestmark = pytest.mark.gpu
@@ -111,3 +111,20 @@ def test_fp32_k_major_tiles(spec):
     o = oracle_run(case, g["logits"], d_aux=0.01, d_z=0.001)
     _routing_equal(g, o)
     _check(case, g, o, 1e-5)
+
+
+def test_fp32_dense_weight_gradients_sum_in_chunks():
+    """The shared expert's gate and up gradients at M = 680, N = 776, T = 1999 are three
+    partial sums over 672 tokens, not one chain of 1999: with every token alike but the
+    first, whose terms are 2^26 times the others' q, the first one's sum loses each q added
+    to it (q is below 1/4 of its ulp), the other two lose none.  At most 671 of 2^26 + 1998
+    are lost (1.0e-5; the terms themselves are 1e-6 off), 1998 in one chain (3.0e-5)."""
+    T, H, S = 1999, 776, 680
+    case = Case(T=T, H=H, E=2, k=1, I=8, S=S, w_std=0.1, seed=3)
+    x = np.tile(case.p["x"][:1], (T, 1))
+    dout = np.tile(case.p["dout"][:1], (T, 1))
+    dout[0] *= 2.0 ** 26
+    g = gpu_run(case, x=x, dout=dout)
+    o = oracle_run(case, g["logits"], x=x, dout=dout)
+    for n in ("shared_gate", "shared_up"):
+        assert rel(g[n], o[n]) <= 671 / 2 ** 26 + 2e-6, n
