@@ -1685,11 +1685,12 @@ __global__ __launch_bounds__(C::THREADS) void k_gateup_dgrad(const T* __restrict
 template <typename T, int NA>
 using WgradTiling = typename std::conditional<NA == 2, typename Tilings<T>::WgradPair,
                                               typename Tilings<T>::Big>::type;
-template <typename T, int NA, bool GROUPED, class C>
+template <typename T, int NA, bool GROUPED>
 MOE_DEV void wgrad_tile(T* smem, int blk, const T* __restrict__ P0, const T* __restrict__ P1,
                         int64_t ldp, const T* __restrict__ Q, int64_t ldq, const KGroups& groups,
                         int M, int N, float alpha, T* const* out0_tab, T* out0_one,
                         T* const* out1_tab, T* out1_one, float* __restrict__ partial) {
+  using C = WgradTiling<T, NA>;
   int grp, split, krow0, K, m0, n0;
   if (!resolve_k(groups, blk, M, N, C::BM, C::BN, grp, split, krow0, K, m0, n0)) return;
   OpDesc<T> a[NA];
@@ -1758,14 +1759,15 @@ MOE_DEV void wgrad_tile(T* smem, int blk, const T* __restrict__ P0, const T* __r
 // dealt over all XCDs instead (skewed counts), tiles of very different K
 // would land unevenly on a static schedule, and the hardware's dispatch
 // balances them better.
-template <typename T, int NA, bool GROUPED, class C = WgradTiling<T, NA>>
-__global__ __launch_bounds__(C::THREADS) void k_wgrad(const T* __restrict__ P0, const T* __restrict__ P1,
+template <typename T, int NA, bool GROUPED>
+__global__ __launch_bounds__((WgradTiling<T, NA>::THREADS)) void k_wgrad(const T* __restrict__ P0, const T* __restrict__ P1,
                                                int64_t ldp, const T* __restrict__ Q, int64_t ldq,
                                                KGroups groups, int M, int N, float alpha,
                                                T* const* out0_tab, T* out0_one,
                                                T* const* out1_tab, T* out1_one,
                                                float* __restrict__ partial, int vblocks,
                                                int slots) {
+  using C = WgradTiling<T, NA>;
   __shared__ __align__(16) T smem[kernel_smem_elems<C, T, NA, 1, NA>()];
   // a grid of `slots` blocks (the host expected whole experts per XCD) runs
   // persistent whatever the flag says; a full grid only when the flag is set
@@ -1773,12 +1775,12 @@ __global__ __launch_bounds__(C::THREADS) void k_wgrad(const T* __restrict__ P0, 
   const bool persist =
       slots > 0 && (reduced || (groups.xcd_order && groups.xcd_order[groups.G]));
   if (!persist) {
-    wgrad_tile<T, NA, GROUPED, C>(smem, (int)blockIdx.x, P0, P1, ldp, Q, ldq, groups, M, N, alpha,
+    wgrad_tile<T, NA, GROUPED>(smem, (int)blockIdx.x, P0, P1, ldp, Q, ldq, groups, M, N, alpha,
                                out0_tab, out0_one, out1_tab, out1_one, partial);
     return;
   }
   for (int vb = (int)blockIdx.x; blockIdx.x < (unsigned)slots && vb < vblocks; vb += slots) {
-    wgrad_tile<T, NA, GROUPED, C>(smem, vb, P0, P1, ldp, Q, ldq, groups, M, N, alpha, out0_tab,
+    wgrad_tile<T, NA, GROUPED>(smem, vb, P0, P1, ldp, Q, ldq, groups, M, N, alpha, out0_tab,
                                out0_one, out1_tab, out1_one, partial);
     __syncthreads();  // the next tile's loads overwrite the epilogue's LDS
   }
@@ -2316,33 +2318,24 @@ MOE_DEV void skinny_rows(f32x4* red, int nb, int r0, int M, const bf16_t* w0, co
   }
 }
 
-// Routed experts (slots: blocks slot by slot, ceil(N / rows of a workgroup)
-// each) or, with slots == nullptr, the dense matrices w0, w1 over M rows of X.
+// Routed experts: blocks slot by slot, ceil(N / rows of a workgroup) each.
 // NC: 1 for batches of at most 16 tokens, else 4.
 template <bool GATEUP, int NC, int KS>
 __global__ __launch_bounds__(256) void k_skinny_fwd(const bf16_t* __restrict__ X,
                                                     const int* __restrict__ xrow, int kdiv,
                                                     int xrows, const SkinnySlot* __restrict__ slots,
-                                                    int M, const bf16_t* w0, const bf16_t* w1,
                                                     int K, int N, bf16_t* __restrict__ out0,
                                                     bf16_t* __restrict__ out1,
                                                     bf16_t* __restrict__ out2) {
   __shared__ f32x4 red[skinny_red<GATEUP, NC, KS, 4>()];
   const int nNb = (N + 16 * (4 / KS) - 1) / (16 * (4 / KS));
   const int slot = uni(blockIdx.x / nNb), nb = uni(blockIdx.x % nNb);
-  int r0 = 0;
-  if (slots) {
-    const SkinnySlot sl = slots[slot];
-    r0 = sl.r0;
-    M = sl.rows;
-    w0 = GATEUP ? sl.gate : sl.down;
-    w1 = sl.up;
-  }
-  if (M <= 0) return;  // workgroup-uniform
-  skinny_rows<GATEUP, NC, KS, 4>(red, nb, uni(r0), uni(M), w0, w1, X, xrow, kdiv, xrows, K, N,
-                                 out0, out1, out2);
+  const SkinnySlot sl = slots[slot];
+  if (sl.rows <= 0) return;  // workgroup-uniform
+  skinny_rows<GATEUP, NC, KS, 4>(red, nb, uni(sl.r0), uni(sl.rows), GATEUP ? sl.gate : sl.down,
+                                 sl.up, X, xrow, kdiv, xrows, K, N, out0, out1, out2);
 }
-// Blocks of a launch over ng slots (or one dense problem).
+// Blocks of a launch over ng slots.
 template <int KS>
 inline int skinny_grid(int ng, int N) { return ng * ((N + 16 * (4 / KS) - 1) / (16 * (4 / KS))); }
 

@@ -578,7 +578,7 @@ struct SmallExtra {
 int small_slots(const moe_config& c, int64_t T) {
   return (int)std::min<int64_t>(c.num_experts, T * c.experts_per_tok);
 }
-template <int EPL, int NC, typename D>
+template <int EPL, int NC>
 void launch_small_route(moe_plan* p, hipStream_t s, int T, char* saved, const SavedLayout& L,
                         const SmallExtra& x) {
   const moe_config& c = p->cfg;
@@ -621,8 +621,8 @@ moe_status run_routing(moe_plan* p, hipStream_t s, int64_t T64, char* saved, cha
   if (T <= kRouteSmallTokens) {
     StageTimer st(p, s, MOE_STAGE_ROUTE);
     auto go = [&](auto epl) {
-      if (T <= 16) launch_small_route<decltype(epl)::value, 1, D>(p, s, T, saved, L, extra);
-      else launch_small_route<decltype(epl)::value, 4, D>(p, s, T, saved, L, extra);
+      if (T <= 16) launch_small_route<decltype(epl)::value, 1>(p, s, T, saved, L, extra);
+      else launch_small_route<decltype(epl)::value, 4>(p, s, T, saved, L, extra);
     };
     switch (route_epl(E)) {
       case 1: go(std::integral_constant<int, 1>()); break;
@@ -950,7 +950,7 @@ void with_row_tiling(const int* offsets, const int* tprefix_all, int E, int64_t 
 // then writes perm and inv_perm.
 template <typename D>
 moe_status routed_fwd(moe_plan* p, hipStream_t s, int T, const D* x, const State<D>& st,
-                      bool timed, const int* gbase = nullptr, const SkinnySlot* slots = nullptr) {
+                      bool timed, const int* gbase, const SkinnySlot* slots) {
   using CG = typename Tilings<D>::GateUp;
   using CB = typename Tilings<D>::Big;
   const moe_config& c = p->cfg;
@@ -960,6 +960,7 @@ moe_status routed_fwd(moe_plan* p, hipStream_t s, int T, const D* x, const State
   // few tokens: no expert holds more than T rows, stream the weights of the
   // experts that the routing listed in `slots` instead
   const bool skinny = std::is_same<D, bf16_t>::value && T <= kSkinnyMaxTokens;
+  if (skinny && !slots) return fail(MOE_ERR_INVALID, "small batch without a list of its experts");
   if (gbase) {  // the dispatch's last launch
     StageTimer tm(p, s, stage(MOE_STAGE_DISPATCH));
     hipLaunchKernelGGL(k_scatter_groups, dim3(ceil_div(T, 4)), dim3(256), 0, s, st.idx, T, k, E,
@@ -976,7 +977,7 @@ moe_status routed_fwd(moe_plan* p, hipStream_t s, int T, const D* x, const State
       auto go = [&](auto nc) {
         hipLaunchKernelGGL((k_skinny_fwd<true, decltype(nc)::value, KS>),
                            dim3(skinny_grid<KS>(small_slots(c, T), I)), dim3(256), 0, s,
-                           (const bf16_t*)x, st.perm, k, T, slots, 0, nullptr, nullptr, H, I,
+                           (const bf16_t*)x, st.perm, k, T, slots, H, I,
                            (bf16_t*)st.G, (bf16_t*)st.U, (bf16_t*)st.A);
       };
       if (T <= 16) go(std::integral_constant<int, 1>());
@@ -999,8 +1000,8 @@ moe_status routed_fwd(moe_plan* p, hipStream_t s, int T, const D* x, const State
       auto go = [&](auto nc) {
         hipLaunchKernelGGL((k_skinny_fwd<false, decltype(nc)::value, KS>),
                            dim3(skinny_grid<KS>(small_slots(c, T), H)), dim3(256), 0, s,
-                           (const bf16_t*)st.A, nullptr, 1, 0, slots, 0, nullptr, nullptr, I,
-                           H, (bf16_t*)st.Y, nullptr, nullptr);
+                           (const bf16_t*)st.A, nullptr, 1, 0, slots, I, H, (bf16_t*)st.Y,
+                           nullptr, nullptr);
       };
       if (T <= 16) go(std::integral_constant<int, 1>());
       else go(std::integral_constant<int, 4>());
