@@ -239,9 +239,11 @@ moe_status moe_saved_field_range(const moe_plan* plan, int64_t num_tokens, int32
 /* Per-stage device timing with HIP events recorded on the call's stream
  * around each stage whose bit (1 << moe_stage) is set in stage_mask; -1 times
  * every stage, 0 (the default) none.  A stage whose work rides another's launch
- * records nothing: the losses (in the combine), and for at most 64 bf16 tokens
- * the dispatch (in the routing) and the shared expert (beside the router GEMM
- * and the routing). */
+ * records nothing.  Above 64 tokens: the losses (in the combine), and where the
+ * router GEMM's launches also route (at most 64 experts, or 256 with hidden
+ * >= 3584) the routing.  Up to 64 tokens: the dispatch and the losses
+ * (in the routing), and in a bf16 forward the shared expert (beside the router
+ * GEMM and the routing). */
 typedef enum {
   MOE_STAGE_ROUTER_GEMM = 0, MOE_STAGE_ROUTE, MOE_STAGE_DISPATCH, MOE_STAGE_GATHER,
   MOE_STAGE_GATEUP_FWD, MOE_STAGE_DOWN_FWD, MOE_STAGE_SHARED_FWD, MOE_STAGE_COMBINE_FWD,

@@ -601,7 +601,7 @@ void launch_small_route(moe_plan* p, hipStream_t s, int T, char* saved, const Sa
 // dispatch.  With `routed` (T > kRouteSmallTokens) the dispatch stops after
 // k_scan: the caller writes perm and inv_perm (k_scatter_groups from the
 // group bases at W.gbase).  The probabilities' column partials ride k_scan; P
-// itself and the losses ride the combine (loss_args).  Up to kRouteSmallTokens
+// itself and the losses ride the combine (LossArgs).  Up to kRouteSmallTokens
 // tokens everything is one launch (k_small_route, with `extra`).
 template <typename D>
 moe_status run_routing(moe_plan* p, hipStream_t s, int64_t T64, char* saved, char* ws,
@@ -634,11 +634,11 @@ moe_status run_routing(moe_plan* p, hipStream_t s, int64_t T64, char* saved, cha
     LAUNCH_CHECK();
     return MOE_OK;
   }
-  {
+  if (!routed) {
     StageTimer st(p, s, MOE_STAGE_ROUTE);
     const int grid = ceil_div(T, 4);
     const float tau = c.router_temperature;
-    if (!routed) switch (route_epl(E)) {
+    switch (route_epl(E)) {
       case 1: launch_route<1>(s, grid, logits, T, E, k, tau, c.norm_topk_prob, probs, lse, idx, w); break;
       case 2: launch_route<2>(s, grid, logits, T, E, k, tau, c.norm_topk_prob, probs, lse, idx, w); break;
       case 4: launch_route<4>(s, grid, logits, T, E, k, tau, c.norm_topk_prob, probs, lse, idx, w); break;

@@ -800,3 +800,32 @@ def test_refused_table_leaves_the_plan_usable():
     g2 = gpu_run(case2, backward=False)
     np.testing.assert_array_equal(second.cpu().numpy(), g2["out"])
     assert not np.array_equal(first.cpu().numpy(), second.cpu().numpy())
+
+
+@pytest.mark.parametrize("spec,route,dispatch,shared", [
+    # the router's launch routes too (fused; split): its k_scan and scatter, no routing stage
+    (dict(T=200, H=64, E=16, k=2, I=32, S=16, dtype="bf16"), 0, 2, 1),
+    (dict(T=65, H=64, E=8, k=2, I=32, S=16, dtype="f32"), 0, 2, 1),
+    (dict(T=130, H=3584, E=72, k=2, I=16, S=0, dtype="bf16"), 0, 2, 0),
+    # a router GEMM, then the routing
+    (dict(T=200, H=64, E=72, k=2, I=32, S=16, dtype="bf16"), 1, 1, 1),
+    # up to 64 tokens one launch routes and dispatches; bf16: the shared expert beside it
+    (dict(T=64, H=64, E=16, k=2, I=32, S=16, dtype="bf16"), 1, 0, 0),
+    (dict(T=64, H=64, E=16, k=2, I=32, S=16, dtype="f32"), 1, 0, 1),
+])
+def test_stages_record_launches_only(spec, route, dispatch, shared):
+    """A stage that rides another's launch records no interval (moe_plan_set_profiling)."""
+    case = Case(**spec, w_std=0.05)
+    dev = torch.device("cuda:0")
+    t = {n: torch.tensor(v, device=dev).to(case.tdtype) for n, v in case.p.items()}
+    plan = Plan(case.cfg, case.tdtype, dev)
+    sh = (t["shared_gate"], t["shared_up"], t["shared_down"]) if case.S else None
+    w, _k = plan.weights_struct(t["router"], *(list(t[n].unbind(0)) for n in ("gate", "up", "down")),
+                                None, sh)
+    plan.set_profiling(None)
+    plan.forward(t["x"], w, need_grad=False)
+    calls = {n: c for n, (_, c) in plan.stage_times().items()}
+    want = dict.fromkeys(calls, 0)
+    want.update(router_gemm=1, route=route, dispatch=dispatch, gateup_fwd=1, down_fwd=1,
+                shared_fwd=shared, combine_fwd=1)
+    assert calls == want
