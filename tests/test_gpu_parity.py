@@ -20,6 +20,7 @@ from oxidizr_amd import _lib
 from oxidizr_amd.moe import MoeConfig, MoeLayer, Plan
 from oxidizr_amd.synth import zipf_bias
 from tests.gpu_helpers import Case, gpu_block_run, gpu_run, oracle_run, rel, rounded
+from tests.tiling_rule import routed
 
 pytestmark = pytest.mark.gpu
 
@@ -140,10 +141,9 @@ BF16_CASES = [
     dict(T=384, H=128, E=64, k=6, I=64, S=128, skew=3.0),
     dict(T=256, H=256, E=256, k=8, I=128, S=128),
     dict(T=200, H=192, E=20, k=4, I=88, S=0, bias=True, norm_topk=True),
-    # >= 512 rows per expert: the row-grouped GEMMs run half-height tail tiles
-    # after every full tile (the tail order of configs 2 and 3)
-    dict(T=1300, H=128, E=4, k=3, I=96, S=32, bias=True, half_last=True),
-    dict(T=1280, H=136, E=4, k=2, I=200, S=0, half_last=True),
+    # >= 512 rows for each of a few experts: 64-row tiles
+    dict(T=1300, H=128, E=4, k=3, I=96, S=32, bias=True),
+    dict(T=1280, H=136, E=4, k=2, I=200, S=0),
     # k above 8: dx's gathers sized for k <= 16
     dict(T=160, H=64, E=12, k=10, I=48, S=16),
     # fused router with a partial last expert block (E = 40) and router bias
@@ -173,7 +173,6 @@ BF16_CASES = [
 def test_bf16_forward_backward_parity(spec):
     spec = dict(spec)
     skew = spec.pop("skew", None)
-    half_last = spec.pop("half_last", False)
     bias = None
     if skew is not None:
         bias = zipf_bias(spec["E"], s=1.2, beta=skew)
@@ -185,50 +184,37 @@ def test_bf16_forward_backward_parity(spec):
     _routing_equal(g, o)
     if skew is not None:
         assert (g["counts"] == 0).any(), "skewed case should leave some experts empty"
-    if half_last:  # the case must hold both kinds of last row tile (256-row tiles)
-        counts = np.asarray(g["counts"])
-        assert spec["T"] * spec["k"] >= 512 * spec["E"]
-        tails = counts % 256
-        assert ((tails > 0) & (tails <= 128)).any() and (tails > 128).any(), counts
     _check(case, g, o, 1e-2)
 
 
-TALL_CASES = [
-    # E = 2, k = 2: every expert receives all T tokens, so the counts are T.
-    # 300 and 320 rows: one 256-row tile that also takes the 44 / 64-row tail
-    # (tall tile); 321: the tail (65 rows) keeps its own tile.
+FEW_GROUP_CASES = [
+    # E = 2, k = 2: every expert receives all T tokens, so the counts are T.  A
+    # last row tile of 44, 64, 1, 30, 64 and 48 rows of 64; I = 296 leaves a
+    # last column tile of 40 (the input gradient of the down projection runs it
+    # at full width)
     dict(T=300, H=128, E=2, k=2, I=96, S=0),
     dict(T=320, H=320, E=2, k=2, I=296, S=32),
     dict(T=321, H=128, E=2, k=2, I=64, S=0),
-    # 350 and 384 rows (tails of 94 and 128 rows, group by group): the full
-    # tile and the tail run as two 192-row tiles (192 + 158, 192 + 192)
     dict(T=350, H=136, E=2, k=2, I=88, S=16),
     dict(T=384, H=128, E=2, k=2, I=64, S=0),
-    # 560 rows = 2 x 256 + 48 with >= 512 rows per expert (tails run last):
-    # the second full tile is tall; I = 296 leaves a last column tile of 40
-    # (the input gradient of the down projection runs it at full width)
     dict(T=560, H=136, E=2, k=2, I=296, S=0),
-    # random counts around 300 rows (some merged tails, some not), router bias
+    # random counts around 300 rows, router bias
     dict(T=1200, H=128, E=8, k=2, I=88, S=16, bias=True),
 ]
 
 
-@pytest.mark.parametrize("spec", TALL_CASES)
-def test_bf16_tall_tile_parity(spec):
-    """Row groups whose last full 256-row tile also takes a tail of at most 64
-    rows (one 320-row tile instead of a full and a quarter tile)."""
+@pytest.mark.parametrize("spec", FEW_GROUP_CASES)
+def test_bf16_few_groups_parity(spec):
+    """A few experts of hundreds of rows leave CUs idle on 256-row tiles and run on 64-row
+    ones (the 256-row tiles at these counts: test_gpu_tilings.test_full_tile_edges)."""
     spec = dict(spec)
     bias = zipf_bias(spec["E"], beta=0.3) if spec.pop("bias", False) else None
+    for gemm in ("gateup", "down", "ddgrad", "gdgrad"):
+        assert routed(spec, gemm) == "small", gemm
     case = Case(**spec, dtype="bf16", w_std=0.05, bias=bias)
     g = gpu_run(case, d_aux=0.01, d_z=0.001)
     o = oracle_run(case, g["logits"], d_aux=0.01, d_z=0.001)
     _routing_equal(g, o)
-    counts = np.asarray(g["counts"])
-    merged = (counts > 256) & (counts % 256 > 0) & (counts % 256 <= 64)
-    if spec["T"] in (321, 350, 384):
-        assert not merged.any(), counts
-    else:
-        assert merged.any(), counts
     _check(case, g, o, 1e-2)
 
 
@@ -300,7 +286,7 @@ SKINNY_CASES = [
     dict(T=48, H=256, E=32, k=4, I=96, S=64),
     dict(T=64, H=136, E=4, k=4, I=40, S=0),        # every expert gets all 64 tokens
     dict(T=7, H=72, E=6, k=2, I=24, S=16),
-    dict(T=64, H=200, E=8, k=2, I=72, S=24),       # ~16 rows per expert: both kernels
+    dict(T=64, H=200, E=8, k=2, I=72, S=24),       # ~16 rows per expert: one chunk or two
 ]
 
 
@@ -334,14 +320,19 @@ def test_bitwise_reproducible(dtype):
 
 
 @pytest.mark.parametrize("dtype,S,E", [("f32", 128, 16), ("bf16", 128, 16), ("bf16", 0, 16),
-                                       ("bf16", 64, 2)])
+                                       ("bf16", 64, 2), ("bf16", 64, 32)])
 def test_shared_stream_overlap_is_bitwise_serial(dtype, S, E):
     # the shared expert on the plan's second stream and the weight gradients
-    # (and the forward's mean probabilities and losses) on its third give the
-    # same bits as the serial order: no result depends on how the streams
-    # interleave.  E = 2: 640 rows per expert, so the row-grouped GEMMs also
-    # run their half-height tiles last.
-    case = Case(T=640, H=128, E=E, k=2, I=64, S=S, dtype=dtype, w_std=0.05, seed=5)
+    # on its third give the same bits as the serial order: no result depends
+    # on how the streams interleave.  E = 32: about 575 rows per expert, so the
+    # row-grouped GEMMs run 256-row tiles, the half-height ones last.
+    T, H, k, I = (640, 128, 2, 64) if E < 32 else (18400, 264, 1, 264)
+    spec = dict(T=T, H=H, E=E, k=k, I=I, S=S)
+    if E == 32:
+        assert T * k >= 512 * E
+        for gemm in ("gateup", "down", "ddgrad", "gdgrad"):
+            assert routed(spec, gemm) == "big", gemm
+    case = Case(**spec, dtype=dtype, w_std=0.05, seed=5)
     a = gpu_run(case, d_aux=0.01, d_z=0.001, overlap=True)
     b = gpu_run(case, d_aux=0.01, d_z=0.001, overlap=False)
     c = gpu_run(case, d_aux=0.01, d_z=0.001, overlap=2)  # shared-expert stream only

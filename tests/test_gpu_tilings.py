@@ -1,47 +1,14 @@
 """The tilings that a launch picks by its size: the shorter ones at the sizes where
 each is picked, and the 256-row family (tall and tail tiles) in launches that fill the CUs,
 which small problems no longer reach."""
-import math
-
 import numpy as np
 import pytest
 
 from tests.gpu_helpers import Case, gpu_run, oracle_run, rel
 from tests.test_gpu_parity import _check, _routing_equal
+from tests.tiling_rule import dense, group_tiles, routed
 
 pytestmark = pytest.mark.gpu
-
-
-def _group_tiles(E, rows, bm):
-    return E * max(1.0, rows / E / bm + 0.5)
-
-
-def _round_cost(tiles, one, two):
-    full, rest = divmod(tiles, 512)
-    return full * two + (0 if rest == 0 else one if rest <= 256 else two)
-
-
-def _leaves_idle(spec, gemm):
-    T, H, E, k, I, S = (spec[n] for n in ("T", "H", "E", "k", "I", "S"))
-    bn = 128 if gemm == "gateup" else 256
-    cols = -(-(H if gemm == "down" else I) // bn)
-    sh = -(-(H if gemm == "down" else S) // bn) if S else 0
-    tiles = _group_tiles(min(E, T * k), T * k, 256) * cols + -(-T // 256) * sh
-    return tiles < 200 and (T * k * cols + T * sh) / 256 < 110
-
-
-def _pick(gateup, N, tiles_of, margin, swiglu_bwd=False):
-    """The rule of with_dense_tiling / with_row_tiling (csrc/moe_api.hip) for a pair that
-    leaves CUs idle; tiles_of(bm): row tiles."""
-    big, mid, small = ((10, (5.2, 7.0), (3.1, 4.7)) if gateup else
-                       (12, (6.8, 8.2), (5.0, 6.2)) if swiglu_bwd else
-                       (10, (6.8, 8.2), (4.4, 5.7)))
-    bn = (128, 64, 64) if gateup else (256, 128, 128)
-    cols = [-(-N // b) for b in bn]
-    cost = {"big": math.ceil(tiles_of(256) * cols[0] / 256) * big / margin,
-            "mid": _round_cost(tiles_of(128) * cols[1], *mid),
-            "small": _round_cost(tiles_of(64) * cols[2], *small)}
-    return min(cost, key=cost.get)
 
 
 PICK_CASES = [
@@ -60,13 +27,8 @@ PICK_CASES = [
 
 @pytest.mark.parametrize("what,tiling,spec", PICK_CASES)
 def test_shorter_tilings(what, tiling, spec):
-    T, E, k = spec["T"], spec["E"], spec["k"]
-    assert _leaves_idle(spec, what[1])
-    dense, gemm = what[0] == "dense", what[1]
-    N = {"gateup": spec["S" if dense else "I"], "ddgrad": spec["S" if dense else "I"],
-         "down": spec["H"]}[gemm]
-    tiles = (lambda bm: -(-T // bm)) if dense else (lambda bm: _group_tiles(E, T * k, bm))
-    assert _pick(gemm == "gateup", N, tiles, 1.0 if dense else 1.15, gemm == "ddgrad") == tiling
+    where, gemm = what
+    assert (dense if where == "dense" else routed)(spec, gemm) == tiling
     # 1e-2: the bf16 bar; the oracle is fp64 on the same bf16 inputs
     case = Case(**spec, dtype="bf16", w_std=0.05)
     g = gpu_run(case, d_aux=0.01, d_z=0.001)
@@ -80,7 +42,7 @@ def test_full_tiles_over_many_experts(T, H, I):
     # 160 experts of about 275, 350 and 562 rows: more than 200 256-row tiles in every
     # routed launch, so the 256-row tilings run, with every kind of tail among the experts
     E, k = 160, 2
-    assert _group_tiles(E, T * k, 256) >= 200
+    assert group_tiles(E, T * k, 256) >= 200
     case = Case(T=T, H=H, E=E, k=k, I=I, S=0, dtype="bf16", w_std=0.05)
     g = gpu_run(case, d_aux=0.01, d_z=0.001)
     o = oracle_run(case, g["logits"], d_aux=0.01, d_z=0.001)
@@ -90,6 +52,40 @@ def test_full_tiles_over_many_experts(T, H, I):
     assert ((counts > 256) & (tails > 0) & (tails <= 64)).any(), counts   # tall tiles
     assert ((counts > 256) & (tails > 64) & (tails <= 128)).any(), counts
     assert (tails > 192).any(), counts
+    _check(case, g, o, 1e-2)
+
+
+# Rows per expert at the edges of the 256-row tilings: a full tile that takes a tail of at
+# most 64 rows (257, 300, 320: one tall tile), tails that keep their own (321, 448, 449, 511),
+# tails of 94 and 128 rows (350, 384: two 192-row tiles), less than a tile (70, 128), whole
+# tiles; then the same behind two full tiles, where the half tiles run last.
+EDGE_ROWS = [300, 320, 321, 350, 384, 256, 257, 70, 385, 448, 449, 511, 128, 512, 576, 640]
+HALF_LAST_ROWS = [560, 576, 577, 640, 641, 700, 512, 513, 767, 768, 300, 320, 600, 832, 448, 400]
+EDGE_CASES = [(EDGE_ROWS * 3, 264, 264), (EDGE_ROWS * 3, 328, 296), (HALF_LAST_ROWS * 2, 264, 264),
+              (HALF_LAST_ROWS * 2, 296, 392)]
+
+
+def _edge_spec(counts, H, I):
+    return dict(T=sum(counts), H=H, E=len(counts), k=1, I=I, S=0)
+
+
+@pytest.mark.parametrize("counts,H,I", EDGE_CASES)
+def test_full_tile_edges(counts, H, I):
+    # H and I of at least five k-tiles: the loops refill their stages in every launch
+    spec = _edge_spec(counts, H, I)
+    T, E = spec["T"], spec["E"]
+    assert (T >= 512 * E) == (counts[0] == HALF_LAST_ROWS[0])  # half tiles last
+    for gemm in ("gateup", "down", "ddgrad", "gdgrad"):
+        assert routed(spec, gemm) == "big", gemm
+    case = Case(**spec, dtype="bf16", w_std=0.05)
+    # token t goes to expert e: logit e is x[t, e], 8 against N(0, 1)
+    expert = np.random.default_rng(0).permutation(np.repeat(np.arange(E), counts))
+    case.p["router"] = np.eye(E, H, dtype=np.float32)
+    case.p["x"][np.arange(T), expert] = 8.0
+    g = gpu_run(case, d_aux=0.01, d_z=0.001)
+    assert list(g["counts"]) == counts
+    o = oracle_run(case, g["logits"], d_aux=0.01, d_z=0.001)
+    _routing_equal(g, o)
     _check(case, g, o, 1e-2)
 
 
