@@ -247,8 +247,9 @@ static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 struct moe_plan {
   moe_config cfg;
   int device;
-  // workgroups of a persistent grouped weight-gradient launch: one per CU
-  // (its tilings hold one workgroup per CU), rounded down to whole XCD rounds
+  // workgroups of a persistent grouped weight-gradient launch: one per CU,
+  // rounded down to whole XCD rounds (the bf16 tilings hold one workgroup per
+  // CU; a CU would hold four of the fp32 pair's)
   int wgrad_slots = 256;
   void* scratch_ptr = nullptr;  // device address of `scratch` on this plan's device
   // device pointer tables: 0 gate, 1 up, 2 down (weights); 3..5 their grads
@@ -759,9 +760,9 @@ struct State {
 //   128 x 128     one 0.6-0.72, two 0.72-0.86    (down 0.83, 1.0 us)
 //   64 x 128      one 0.31-0.48, two 0.51-0.59   (down 0.40, 0.69 us)
 //   gate/up 128 x 64: 0.5-0.55, 0.7;  64 x 64: 0.30, 0.47
-// T = 500, H = 2048, S = 2816 alone, 256-row tiles -> picked: gate/up forward 44
-// -> 22 us, down 50 -> 18, down input gradient 60 -> 27, gate/up input gradient
-// 127 -> 61.  An experts' launch counts its rows as evenly spread (an expert's
+// T = 500, H = 2048, S = 2816 alone, 256-row tiles -> the cheapest: gate/up
+// forward 44 -> 22 us, down 50 -> 18, down input gradient 60 -> 27, gate/up input
+// gradient 127 -> 61.  An experts' launch counts its rows as evenly spread (an expert's
 // last tile half empty on average) and changes only for an estimated gain of 15
 // %: weights that stream from memory set the time of launches with few rows per
 // expert, whatever the tile.  Alone, 16 experts of 62 rows (H = 2048, I = 1408):
@@ -771,14 +772,20 @@ struct State {
 // The shorter tilings take more CU time for the same work, so they pay only
 // while a routed launch and the shared expert's beside it leave CUs idle: below
 // kBusyTiles 256-row tiles in both, that hold fewer rows than kBusyRows full
-// ones (leaves_idle).  Steps (fwd + bwd, E = 16, k = 2, H = 2048, I = 1408, S =
-// 2816): T = 300 481 -> 366 us, 500 543 -> 412, 750 557 -> 452, 1000 550 -> 504,
-// 1250 599 -> 592, 2000 unchanged; forward T = 500 166 -> 137; without a shared
-// expert T = 2000 463 -> 433.  Fewer tiles (130, 160) lose most of it (T = 500
-// 503, T = 1000 552), more (260) cost T = 2000 662 -> 716, no limit costs T =
-// 1500, E = 64, k = 6 forward 369 -> 389.  More full rows (130) cost T = 2646, H =
-// 840, E = 8, I = S = 1936 559 -> 568 (its dense tiles are full), fewer (90) lose
-// T = 1000.
+// ones (leaves_idle).  us, no shorter tiling -> this rule; steps of E = 16, k = 2, H
+// = 2048, I = 1408, S = 2816: T = 300 451 -> 354, 500 508 -> 391, 750 537 -> 433,
+// 1000 547 -> 498 (from T = 1250 on it takes none); forward T = 500 158 -> 113;
+// without a shared expert T = 2000 438 -> 410.  Slower with it: E = 32, k = 4, H =
+// 1024, I = S = 1536, T = 600 394 -> 410.
+// Other kBusyTiles: 130 loses most of it (T = 300 419, 500 488, 750 500, 1000
+// 545), 160 less (T = 1000 538); 230 and more also give the gate/up forward of
+// small T the short tiles (220 tiles at T = 500), for better and worse: forward T =
+// 300 106 -> 93, T = 500 113 -> 124, steps 354 -> 345 and 391 -> 396, others the
+// same.  Other kBusyRows: 90 loses T = 1000 (540) and the T = 2000 without a shared
+// expert (440); 130 costs E = 8, k = 2, H = 4096, I = S = 1536, T = 600 458 -> 490
+// (T = 1250 above 578 -> 569).  Neither limit: T = 2000 640 -> 728, forward of T =
+// 1500, E = 64, k = 6 358 -> 381, though T = 2646, E = 8, k = 2, H = 840, I = S = 1936
+// 543 -> 517.
 constexpr double kBusyTiles = 200, kBusyRows = 110;
 struct TileCost {
   double one, two;
@@ -818,8 +825,10 @@ bool leaves_idle(const moe_config& c, int64_t T, int n_routed, int n_shared, int
 // rows and N columns: C, its 384-row tiles or one of the shorter tilings,
 // whichever costs least.  The last row tile of C or its 384-row tiles runs as
 // the shortest tiling that covers it.  idle: leaves_idle of it and the routed
-// launch beside it.  MID = false (the launches over H columns): such a launch
-// that leaves CUs idle holds at most 440 64 x 128 tiles, fewer than a round.
+// launch beside it.  MID = false (the launches over H columns): no 128 x 128
+// tiles.  Up to H = 8192 such a launch that leaves CUs idle holds at most 496
+// 64 x 128 tiles (T = 454): one round of two to a CU, which costs less than any
+// round of the others.  Wider layers have up to 594 (H = 25344, T = 133).
 template <typename D, class C, bool MID, class F>
 void with_dense_tiling(int T, int N, const TileCosts& cost, bool idle, F&& f) {
   auto tiles = [&](auto c) {
