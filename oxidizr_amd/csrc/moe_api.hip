@@ -203,7 +203,8 @@ SplitPlan plan_split(int M, int N, int K) {
 // tiles of 32-deep ones: the cost model has one workgroup to a CU, and on the
 // launch's own tile it splits less (a tenth of the shapes with M and N up to some
 // thousands).  M = 680, N = 776, T = 1999: 1 chunk instead of 3, and gradients
-// 7.9e-7 off a 64-bit sum instead of 4.6e-7.
+// 7.9e-7 off a 64-bit sum instead of 4.6e-7 (69 us alone; with 3 chunks 49, and 5
+// for their sum).
 template <typename D, int NA>
 SplitPlan plan_dense_wgrad(int M, int N, int T) {
   using C = WgradTiling<D, NA>;
