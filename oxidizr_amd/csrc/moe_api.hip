@@ -172,7 +172,10 @@ void norm_tree(int nrow, F&& level) {
 // per chunk, plus, when split, the fp32 partial tiles written and read back by
 // k_splitk_reduce (8 bytes per output element and chunk at ~5 TB/s, against
 // ~3.9 TFLOP/s of MFMA work per CU: 3.1 * M * N / (BM * BN * BK) units per
-// chunk).  The split depends only on the shapes, never on timing.
+// chunk).  These are the bf16 tilings' rates; fp32 does ~0.6 TFLOP/s per CU and
+// holds several workgroups there, so its chunks are priced some six times too
+// high and it splits less than would be fastest (M = 776, N = 680, T = 1999: one
+// chunk, 144 workgroups).  The split depends only on the shapes, never on timing.
 struct SplitPlan {
   int nsplit, kchunk;
 };
